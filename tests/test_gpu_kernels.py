@@ -89,6 +89,21 @@ def test_router_ids_bit_exact(dev, m):
     np.testing.assert_allclose(w.cpu().numpy(), rw, rtol=2e-6, atol=0)
 
 
+# the matrix-core form (m > 8): ragged token and expert tiles, the shortest column split, both tile sizes
+@pytest.mark.parametrize("m,n_exp,d,k", [(9, 256, 4096, 6), (17, 160, 512, 4), (33, 1000, 1536, 8),
+                                         (640, 30, 512, 6), (641, 64, 1024, 6), (700, 40, 512, 16)])
+def test_router_many_tokens_bit_exact(dev, m, n_exp, d, k):
+    gate, bias = synthetic.router_weights(m, 0, n_exp, d, dev)
+    x = synthetic.hidden(m, 0, m, d, dev)
+    for _ in range(2):  # the second call finds the arrival counters as the first left them
+        idx, w, lg = ops.router_topk(x, gate, bias, k, 1.5, want_logits=True)
+        ridx, rw, _, rlg = orc.router(orc.to_np_bf16(x), orc.to_np_bf16(gate), bias.cpu().numpy(), k, 1.5,
+                                      return_scores=True)
+        assert np.array_equal(orc.to_np_bf16(lg), rlg)
+        assert np.array_equal(idx.cpu().numpy(), ridx)
+        np.testing.assert_allclose(w.cpu().numpy(), rw, rtol=2e-6, atol=0)
+
+
 def test_router_ties_and_no_bias(dev):
     x = torch.ones(2, 512, dtype=torch.bfloat16, device=dev)
     gate = torch.full((64, 512), 0.5, dtype=torch.bfloat16, device=dev)
