@@ -162,6 +162,7 @@ __global__ void __launch_bounds__(64 * kP2Waves) moe_down_kernel(DecodeParams p)
   __shared__ int s_cand[kMaxCand];
   __shared__ int s_first[kMaxCand];
   __shared__ int s_last;
+  __shared__ bool s_sel[kMaxTok][kMaxCand + 1];
   build_plan(p, plan, s_cand, s_first);
   const int n_slots = plan.n_routed + (p.shared ? 1 : 0);
   const int s = blockIdx.y;
@@ -226,10 +227,19 @@ __global__ void __launch_bounds__(64 * kP2Waves) moe_down_kernel(DecodeParams p)
              (unsigned)(n_slots - 1);
   __syncthreads();
   if (!s_last) return;
+  // the slots a token selects (the shared one: every token); the other slots'
+  // partials of it are products with zero activations and stay out of its sum
+  for (int q = threadIdx.x; q < n_slots * p.m; q += blockDim.x) {
+    const int sl = q / p.m, t = q - sl * p.m;
+    bool sel = sl == plan.n_routed;
+    for (int k = 0; k < p.top_k && !sel; ++k) sel = p.idx[t * p.top_k + k] == plan.eid[sl];
+    s_sel[t][sl] = sel;
+  }
+  __syncthreads();
   const int rows = 16 * kP2Waves;
   for (int q = threadIdx.x; q < rows * p.m; q += blockDim.x) {
     const int t = q / rows, d = blockIdx.x * rows + (q - t * rows);
-    const float v = sum_slots_agent(p.part + (int64_t)t * p.d + d, (int64_t)p.m * p.d, n_slots, nullptr);
+    const float v = sum_slots_agent(p.part + (int64_t)t * p.d + d, (int64_t)p.m * p.d, n_slots, s_sel[t]);
     const int64_t o = (int64_t)t * p.d + d;
     if (p.out_f32) p.out_f32[o] = v;
     if (p.out_bf16) p.out_bf16[o] = (uint16_t)f32_to_bf16_bits(v);

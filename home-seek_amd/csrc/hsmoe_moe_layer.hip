@@ -106,9 +106,9 @@ struct LayerParams {
   unsigned* ctl;
   uint64_t* scores;     // kScoreCopies copies of [m][n_exp] tagged fp32 scores
   int score_stride;     // 64-bit words between copies
-  uint64_t* act;   // tagged [S][m][i] weighted activations of the routed slots
+  uint64_t* act;   // tagged [pairs][i] weighted activations of the routed (slot, token) pairs
   uint64_t* sgh;   // tagged [2][m][i] shared expert gate row sums (0) and activations (1)
-  uint64_t* part;  // tagged [S + 1][m][d] per-slot down partials (slot S: shared)
+  uint64_t* part;  // tagged down partials: [S][d] of the pairs, then [m][d] of the shared expert
   uint64_t* fin;   // tagged [m][d] output rows for the tail items, or null (no tail)
   uint4* wipe;      // the workspace after the control words, zeroed at a re-arm
   int64_t wipe_n;   //   (16-byte units)
@@ -179,26 +179,79 @@ __device__ __forceinline__ void poll_tagged(const uint64_t* ubase, int64_t jstri
   if (need) store_agent(ctl + kCtlErr, 1u + (unsigned)code);
 }
 
-struct Shared {
-  uint64_t ent[kMaxSlots + 1][6];     // table entry of routed slot s (and of the shared expert at slot S)
-  float red[kWaves][2][16 * kMaxTok];  // gate/up partials: [wave][gate|up][row * kMaxTok + token]
-  double rpart[kWaves][kMaxTok];  // router: per-wave partial logit sums
-  float rscore[kMaxTok];          // router: the row's score per token
+// poll_tagged over up to 8 rows of words: rows pair[j] (wave-uniform), `d`
+// words each, base already at the lane's column.
+__device__ __forceinline__ void poll_tagged_pairs(const uint64_t* base, const unsigned char* pair, int d, int cnt,
+                                                  unsigned tag, float (&v)[8], unsigned* ctl, int code) {
+  unsigned need = 0;
+  uint32_t off[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    v[j] = 0.0f;
+    off[j] = 0;
+    if (j < cnt) {
+      need |= 1u << j;
+      off[j] = (uint32_t)__builtin_amdgcn_readfirstlane(pair[j]) * (uint32_t)d;
+    }
+  }
+  for (unsigned it = 0; it < kSpinLimit; ++it) {
+    const unsigned cur = need;
+    uint64_t w[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w[j] = (cur >> j) & 1u ? load_agent(base + off[j]) : 0ull;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (((cur >> j) & 1u) && (unsigned)(w[j] >> 32) == tag) {
+        v[j] = __uint_as_float((unsigned)w[j]);
+        need &= ~(1u << j);
+      }
+    if (__ballot(need != 0) == 0) return;
+    __builtin_amdgcn_s_sleep(2);
+  }
+  if (need) store_agent(ctl + kCtlErr, 1u + (unsigned)code);
+}
+
+// What the slot plan's build works on; its LDS is the items' reduction scratch
+// otherwise (plan_item begins and ends with a barrier).
+struct PlanBuild {
   int64_t idx[kMaxSlots];  // top-k ids of every token
   float w[kMaxSlots];      // top-k weights of every token
-  int eid[kMaxSlots];            // slot plan: expert id of routed slot s
-  float wt[kMaxSlots][kMaxTok];  // slot plan: weight of routed slot s for token t
-  float wt_item[kMaxTok];
+  alignas(4) unsigned char valid[kMaxExperts];  // expert e has a table entry
+  alignas(4) unsigned char used[kMaxExperts];   // expert e is selected by some token
+  short rank[kMaxExperts];                      // slot of a selected expert
+  unsigned char pslot[kMaxSlots];               // slot of top-k entry j (0xff: none, or an id met before)
+};
+
+// The slot plan lists the (slot, token) pairs the routing selects, slots
+// ascending and a slot's tokens ascending: pair u = off[s] + (tokens of the
+// slot before this one).  Only pairs are computed and handed on: a down item
+// stages its slot's pairs' activations, not every token's (at m = 8 a slot has
+// 1.1 pairs on average, and all 8 tokens' tagged words were twice the item's
+// weights), and a row group adds the partials of a token's own slots.
+struct Shared {
+  uint64_t ent[kMaxSlots + 1][6];     // table entry of routed slot s (and of the shared expert at slot S)
+  union {
+    float red[kWaves][2][16 * kMaxTok];  // gate/up partials: [wave][gate|up][row * kMaxTok + token]
+    PlanBuild b;
+  };
+  double rpart[kWaves][kMaxTok];  // router: per-wave partial logit sums
+  float rscore[kMaxTok];          // router: the row's score per token
+  float pw[kMaxSlots];                             // weight of pair u
+  alignas(4) unsigned char tmask[kMaxSlots];       // bit t: token t selects slot s
+  unsigned char off[kMaxSlots];                    // first pair of slot s
+  unsigned char ptok[kMaxSlots];                   // token of pair u
+  unsigned char tpair[kMaxTok][16];                // pairs of token t, slots ascending
+  unsigned char ntp[kMaxTok];                      // how many
   unsigned tag;  // this launch's tag (read_launch_tag, once per workgroup)
-  int flag;
   int n_routed;
   int have_plan;
   int last;  // this workgroup is the last of the launch to finish
-  alignas(4) unsigned char valid[kMaxExperts];  // expert e has a table entry (plan build)
-  alignas(4) unsigned char used[kMaxExperts];   // expert e is selected by some token (plan build)
-  short rank[kMaxExperts];                      // slot of a selected expert (plan build)
 };
 static_assert(sizeof(Shared::red) >= 2 * 64 * 4 * sizeof(float), "shared down: two waves' accumulators");
+// With the largest tile (64 KiB: m = 8 at i = 2048, d = 4096) two workgroups
+// still share a CU's 160 KiB of LDS; at 17.8 KB of scratch they did not, and
+// the launch ran on half the workgroups.
+static_assert(sizeof(Shared) <= 16384 - 256, "two workgroups per CU with a 64 KiB tile");
 
 // The router part of the slot plan: wave w takes the top-k of tokens w,
 // w + kWaves (ties to the lower index) from the tokens' tagged scores, polled
@@ -251,16 +304,16 @@ __device__ __forceinline__ void build_plan_scores(const LayerParams& p, Shared& 
   }
   if (!seen && lane == 0) store_agent(p.ctl + kCtlErr, 1u + (unsigned)kWaitScores);
   // (the table loads were in flight with the first poll)
-  if ((int)threadIdx.x < p.n_exp) sh.valid[threadIdx.x] = my_ent[0] != 0ull;
-  sh.used[threadIdx.x] = 0;  // all kMaxExperts == kThreads bytes: wave 0 reads them as words
+  if ((int)threadIdx.x < p.n_exp) sh.b.valid[threadIdx.x] = my_ent[0] != 0ull;
+  sh.b.used[threadIdx.x] = 0;  // all kMaxExperts == kThreads bytes: wave 0 reads them as words
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     const int t = wave + kWaves * j;
-    if (t < p.m) wave_topk_vals<4>(v[j], p.n_exp, p.top_k, p.scaling, sh.idx + t * p.top_k, sh.w + t * p.top_k);
+    if (t < p.m) wave_topk_vals<4>(v[j], p.n_exp, p.top_k, p.scaling, sh.b.idx + t * p.top_k, sh.b.w + t * p.top_k);
   }
 }
 
-// Slots from sh.idx / sh.w: the distinct valid ids ascending, each token's
+// Slots from sh.b.idx / sh.w: the distinct valid ids ascending, each token's
 // weight of each slot, the slots' table entries.
 __device__ __forceinline__ void finish_plan(const LayerParams& p, Shared& sh, const uint64_t (&my_ent)[6]) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -269,15 +322,14 @@ __device__ __forceinline__ void finish_plan(const LayerParams& p, Shared& sh, co
   // Wave 0 alone (LDS accesses of one wave take effect in program order):
   // mark the selected valid experts, rank them ascending (lane l counts
   // experts 4l .. 4l+3; exclusive prefix of the counts from three ballots),
-  // then each token's weight of each slot (at most one top-k entry, as a
-  // token's ids are distinct; else 0).
+  // then list the (slot, token) pairs and each token's pairs.
   if (wave == 0) {
     for (int j = lane; j < n; j += 64) {
-      const int64_t e = sh.idx[j];
-      if (e >= 0 && e < p.n_exp && sh.valid[e]) sh.used[e] = 1;
+      const int64_t e = sh.b.idx[j];
+      if (e >= 0 && e < p.n_exp && sh.b.valid[e]) sh.b.used[e] = 1;
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    const uint32_t u4 = reinterpret_cast<const uint32_t*>(sh.used)[lane];
+    const uint32_t u4 = reinterpret_cast<const uint32_t*>(sh.b.used)[lane];
     const uint32_t b0 = (u4 & 0xffu) != 0, b1 = (u4 & 0xff00u) != 0, b2 = (u4 & 0xff0000u) != 0,
                    b3 = (u4 & 0xff000000u) != 0;
     const uint32_t c = b0 + b1 + b2 + b3;
@@ -287,40 +339,91 @@ __device__ __forceinline__ void finish_plan(const LayerParams& p, Shared& sh, co
                     4 * (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m2 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m2, 0));
     const int base = __popcll(m0) + 2 * __popcll(m1) + 4 * __popcll(m2);
     const int e4 = 4 * lane;
-    if (b0) { sh.rank[e4] = (short)pre; sh.eid[pre] = e4; }
-    if (b1) { sh.rank[e4 + 1] = (short)(pre + b0); sh.eid[pre + b0] = e4 + 1; }
-    if (b2) { sh.rank[e4 + 2] = (short)(pre + b0 + b1); sh.eid[pre + b0 + b1] = e4 + 2; }
-    if (b3) { sh.rank[e4 + 3] = (short)(pre + b0 + b1 + b2); sh.eid[pre + b0 + b1 + b2] = e4 + 3; }
-    for (int s0 = 0; s0 < base; s0 += 64 / kMaxTok) {  // zero weights: (slot, token) per lane
-      const int sl = s0 + lane / kMaxTok, t = lane % kMaxTok;
-      if (sl < base && t < p.m) sh.wt[sl][t] = 0.0f;
-    }
+    if (b0) sh.b.rank[e4] = (short)pre;
+    if (b1) sh.b.rank[e4 + 1] = (short)(pre + b0);
+    if (b2) sh.b.rank[e4 + 2] = (short)(pre + b0 + b1);
+    if (b3) sh.b.rank[e4 + 3] = (short)(pre + b0 + b1 + b2);
+    reinterpret_cast<uint16_t*>(sh.tmask)[lane] = 0;  // all kMaxSlots == 128 bytes
+    if (lane < kMaxTok) sh.ntp[lane] = 0;
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    if (!p.route_idx) {  // router ids: distinct per token
-      for (int j = lane; j < n; j += 64) {
-        const int64_t e = sh.idx[j];
-        if (e >= 0 && e < p.n_exp && sh.valid[e]) sh.wt[sh.rank[e]][j / p.top_k] = __fadd_rn(0.0f, sh.w[j]);
-      }
-    } else {  // given ids may repeat within a token: their weights add, in k order
-      for (int j = lane; j < n; j += 64) {
-        const int64_t e = sh.idx[j];
-        const int t = j / p.top_k, c0 = t * p.top_k;
-        bool first = e >= 0 && e < p.n_exp && sh.valid[e];
-        for (int c = c0; c < j && first; ++c) first = sh.idx[c] != e;
-        if (first) {
-          float w = 0.0f;
-          for (int c = c0; c < c0 + p.top_k; ++c)
-            if (sh.idx[c] == e) w = __fadd_rn(w, sh.w[c]);
-          sh.wt[sh.rank[e]][t] = w;
+    // the pairs of top-k entries lane and lane + 64 (n <= kMaxSlots): slot
+    // (-1: none) and weight.  Router ids are distinct per token; given ids may
+    // repeat, then the first carries the weights' sum in k order.
+    int sl[2];
+    float wt[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int j = lane + 64 * h;
+      sl[h] = -1;
+      wt[h] = 0.0f;
+      if (j < n) {
+        const int64_t e = sh.b.idx[j];
+        bool first = e >= 0 && e < p.n_exp && sh.b.valid[e];
+        if (!p.route_idx) {
+          wt[h] = __fadd_rn(0.0f, sh.b.w[j]);
+        } else {
+          const int c0 = j / p.top_k * p.top_k;
+          for (int c = c0; c < j && first; ++c) first = sh.b.idx[c] != e;
+          if (first)
+            for (int c = c0; c < c0 + p.top_k; ++c)
+              if (sh.b.idx[c] == e) wt[h] = __fadd_rn(wt[h], sh.b.w[c]);
         }
+        if (first) sl[h] = sh.b.rank[e];
+      }
+    }
+    if (p.m == 1) {  // one token: pair u is slot u
+      if (sl[0] >= 0) {
+        sh.tmask[sl[0]] = 1;
+        sh.ptok[sl[0]] = 0;
+        sh.off[sl[0]] = sh.tpair[0][sl[0]] = (unsigned char)sl[0];
+        sh.pw[sl[0]] = wt[0];
+      }
+      if (lane == 0) sh.ntp[0] = (unsigned char)base;
+    } else {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int j = lane + 64 * h;
+        if (j < n) sh.b.pslot[j] = (unsigned char)sl[h];
+        if (sl[h] >= 0)
+          atomicOr(reinterpret_cast<unsigned*>(sh.tmask) + (sl[h] >> 2), 1u << (8 * (sl[h] & 3) + j / p.top_k));
+      }
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      // first pairs: lane l counts slots 2l and 2l + 1 (at most 16 pairs), the
+      // exclusive prefix of the counts from five ballots
+      const uint32_t mk = reinterpret_cast<const uint16_t*>(sh.tmask)[lane];
+      const int n0 = __popc(mk & 0xffu), nn = __popc(mk);
+      int before = 0;
+#pragma unroll
+      for (int bit = 0; bit < 5; ++bit) {
+        const uint64_t mb = __ballot((nn >> bit) & 1);
+        before += (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mb, 0)) << bit;
+      }
+      sh.off[2 * lane] = (unsigned char)before;
+      sh.off[2 * lane + 1] = (unsigned char)(before + n0);
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (sl[h] < 0) continue;
+        const int j = lane + 64 * h, t = j / p.top_k, c0 = t * p.top_k;
+        const int u = sh.off[sl[h]] + __popc(sh.tmask[sl[h]] & ((1u << t) - 1u));
+        sh.pw[u] = wt[h];
+        sh.ptok[u] = (unsigned char)t;
+        int r = 0, cnt = 0;  // among the token's slots
+        for (int c = c0; c < c0 + p.top_k; ++c) {
+          const int o = sh.b.pslot[c];
+          cnt += o != 0xff;
+          r += o < sl[h];
+        }
+        sh.tpair[t][r] = (unsigned char)u;
+        if (r == 0) sh.ntp[t] = (unsigned char)cnt;
       }
     }
     if (lane == 0) sh.n_routed = base;
   }
   __syncthreads();
   // each selected expert's thread moves its table entry into its slot
-  if ((int)threadIdx.x < p.n_exp && sh.used[threadIdx.x]) {
-    const int sl = sh.rank[threadIdx.x];
+  if ((int)threadIdx.x < p.n_exp && sh.b.used[threadIdx.x]) {
+    const int sl = sh.b.rank[threadIdx.x];
 #pragma unroll
     for (int k = 0; k < 6; ++k) sh.ent[sl][k] = my_ent[k];
   }
@@ -348,11 +451,11 @@ __device__ __forceinline__ void build_plan(const LayerParams& p, Shared& sh, con
       } else {
         e = ldg<int64_t>(p.route_idx + j);
       }
-      sh.idx[j] = e;
-      sh.w[j] = p.route_w ? ldg<float>(p.route_w + j) : p.route_wconst;
+      sh.b.idx[j] = e;
+      sh.b.w[j] = p.route_w ? ldg<float>(p.route_w + j) : p.route_wconst;
     }
-    if ((int)threadIdx.x < p.n_exp) sh.valid[threadIdx.x] = my_ent[0] != 0ull;
-    sh.used[threadIdx.x] = 0;
+    if ((int)threadIdx.x < p.n_exp) sh.b.valid[threadIdx.x] = my_ent[0] != 0ull;
+    sh.b.used[threadIdx.x] = 0;
   } else {
     build_plan_scores(p, sh, my_ent);
   }
@@ -363,8 +466,8 @@ __device__ __forceinline__ void build_plan(const LayerParams& p, Shared& sh, con
 // and no shared expert), written once by the plan builder.
 __device__ __forceinline__ void write_routing(const LayerParams& p, Shared& sh) {
   for (int j = threadIdx.x; j < p.m * p.top_k; j += kThreads) {
-    if (p.idx_out) p.idx_out[j] = sh.idx[j];
-    if (p.w_out) p.w_out[j] = sh.w[j];
+    if (p.idx_out) p.idx_out[j] = sh.b.idx[j];
+    if (p.w_out) p.w_out[j] = sh.b.w[j];
   }
   if (sh.n_routed == 0 && !p.shared) {
     // no down item will run, and the output is zero (_forward_legacy returns
@@ -418,12 +521,16 @@ __device__ __forceinline__ uint64_t* fin_late(uint64_t kernarg) {
 __device__ __noinline__ void plan_item(uint64_t kernarg) {
   const LayerParams p = params(kernarg);
   Shared& sh = g_sh;
+  __syncthreads();  // the previous item's readers of the reduction scratch are done
   uint64_t my_ent[6];  // expert threadIdx.x's table entry
 #pragma unroll
   for (int k = 0; k < 6; ++k)
     my_ent[k] = (int)threadIdx.x < p.n_exp ? ldg<uint64_t>(p.table + (int64_t)threadIdx.x * 6 + k) : 0ull;
   build_plan(p, sh, my_ent);
-  if (blockIdx.x == gridDim.x - 1) write_routing(p, sh);  // read only after the launch
+  if (blockIdx.x == gridDim.x - 1) {
+    write_routing(p, sh);  // read only after the launch
+    __syncthreads();       // the next item rewrites the build's LDS
+  }
 }
 
 // plan_item for given routing when a gate/up item comes next and the LDS
@@ -524,6 +631,11 @@ __device__ __forceinline__ int router_item(uint64_t kernarg, int q_arg, int stat
   return state;
 }
 
+// The pair of slot s and token t (which selects the slot).
+__device__ __forceinline__ int pair_of(const Shared& sh, int s, int t) {
+  return sh.off[s] + __popc(sh.tmask[s] & ((1u << t) - 1u));
+}
+
 __device__ __noinline__ int gate_up_item(uint64_t kernarg, int q_arg, int state_arg) {
   const int q = __builtin_amdgcn_readfirstlane(q_arg);
   int state = __builtin_amdgcn_readfirstlane(state_arg);
@@ -536,7 +648,6 @@ __device__ __noinline__ int gate_up_item(uint64_t kernarg, int q_arg, int state_
   const int r0 = (qq % gu_per_slot) * kGuRows;
   if (s >= sh.n_routed) return state;
   const unsigned tag = g_sh.tag;
-  if (threadIdx.x < p.m) sh.wt_item[threadIdx.x] = sh.wt[s][threadIdx.x];
   const uint64_t* ent = sh.ent[s];
   ensure_x(p, state);
   const int per = (p.d / 128) / kWaves;
@@ -553,15 +664,16 @@ __device__ __noinline__ int gate_up_item(uint64_t kernarg, int q_arg, int state_
   }
   __syncthreads();
   const int row = threadIdx.x >> 4, col = threadIdx.x & 15;
-  if (col < p.m) {
+  if ((sh.tmask[s] >> col) & 1) {
     float gsum = 0.0f, usum = 0.0f;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
       gsum = __fadd_rn(gsum, sh.red[w][0][row * kMaxTok + col]);
       usum = __fadd_rn(usum, sh.red[w][1][row * kMaxTok + col]);
     }
-    const float a = __fmul_rn(sh.wt_item[col], swiglu(gsum, usum, p.limit));
-    store_agent(p.act + ((int64_t)s * p.m + col) * p.i + r0 + row, tagged(tag, __float_as_uint(a)));
+    const int u = pair_of(sh, s, col);
+    const float a = __fmul_rn(sh.pw[u], swiglu(gsum, usum, p.limit));
+    store_agent(p.act + (int64_t)u * p.i + r0 + row, tagged(tag, __float_as_uint(a)));
   }
   return state;
 }
@@ -644,7 +756,6 @@ __device__ __noinline__ int gate_up_run(uint64_t kernarg, int q_arg, int state_a
   b1.load(w1, r0 + r, p.d, st0, g);
   b3.load(w3, r0 + r, p.d, st0, g);
   for (;;) {
-    if (threadIdx.x < p.m) sh.wt_item[threadIdx.x] = sh.wt[s][threadIdx.x];
     f32x4 ag = {0, 0, 0, 0}, au = {0, 0, 0, 0};
     for (int bt = 0; bt < nb; ++bt) {
       const int st = st0 + bt * kB;
@@ -683,18 +794,19 @@ __device__ __noinline__ int gate_up_run(uint64_t kernarg, int q_arg, int state_a
     __syncthreads();
     {
       const int row = threadIdx.x >> 4, col = threadIdx.x & 15;
-      if (col < p.m) {
+      if ((sh.tmask[s] >> col) & 1) {
         float gsum = 0.0f, usum = 0.0f;
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
           gsum = __fadd_rn(gsum, sh.red[w][0][row * kMaxTok + col]);
           usum = __fadd_rn(usum, sh.red[w][1][row * kMaxTok + col]);
         }
-        const float a = __fmul_rn(sh.wt_item[col], swiglu(gsum, usum, p.limit));
-        store_agent(p.act + ((int64_t)s * p.m + col) * p.i + r0 + row, tagged(tag, __float_as_uint(a)));
+        const int u = pair_of(sh, s, col);
+        const float a = __fmul_rn(sh.pw[u], swiglu(gsum, usum, p.limit));
+        store_agent(p.act + (int64_t)u * p.i + r0 + row, tagged(tag, __float_as_uint(a)));
       }
     }
-    __syncthreads();  // sh.red and sh.wt_item are rewritten by the next item
+    __syncthreads();  // sh.red is rewritten by the next item
     if (!next) break;
     q = q2;
     s = s2;
@@ -751,6 +863,11 @@ __device__ __forceinline__ int down_index(const LayerParams& p, int s, int g) {
   return p.d0 + s * dps + g;
 }
 
+// One routed slot, which every token selects, and no shared expert.
+__device__ __forceinline__ bool lone_slot(const LayerParams& p, const Shared& sh) {
+  return sh.n_routed == 1 && !p.shared && sh.tmask[0] == (1u << p.m) - 1u;
+}
+
 // Down item q, first part: W2 rows of the slot against its activations, the
 // slot's fp32 partial sums published (tagged) for the row group.  Needs the
 // slot plan for a routed slot only (the shared slot may run before the plan
@@ -773,9 +890,11 @@ __device__ __noinline__ int down_item(uint64_t kernarg, int q_arg, int state_arg
   // shared: waves 0 and 2 (1 and 3) take rows r0 .. r0 + 15 over the first
   // (second) step range
   const int r0 = kShared ? g * kDownRows + 32 * h + 16 * (wave & 1) : g * kDownRows + 16 * wave;
-  const int m = p.m, i = p.i;
+  // columns: the slot's pairs (shared: every token)
+  const int i = p.i, m = kShared ? p.m : __builtin_amdgcn_readfirstlane(__popc(sh.tmask[s]));
+  const int u0 = kShared ? 0 : __builtin_amdgcn_readfirstlane(sh.off[s]);
   unsigned* const ctl = p.ctl;
-  const uint64_t* const src = p.act + (int64_t)s * m * i;
+  const uint64_t* const src = p.act + (int64_t)u0 * i;
   const uint64_t* const sgh = p.sgh;
   f32x4 acc = {0, 0, 0, 0};
   auto stage = [&]() __attribute__((always_inline)) {
@@ -786,8 +905,8 @@ __device__ __noinline__ int down_item(uint64_t kernarg, int q_arg, int state_arg
     if (!kShared && state == 2 + s) return;
     const int n = m * i;
     constexpr int kStageWords = 8;  // per thread and round (registers: the W2 batch is live)
-    for (int u0 = 0; u0 < n; u0 += kStageWords * kThreads) {  // this thread's words u0 + threadIdx.x + kThreads * j
-      const int c0 = u0 + (int)threadIdx.x;
+    for (int w0 = 0; w0 < n; w0 += kStageWords * kThreads) {  // this thread's words w0 + threadIdx.x + kThreads * j
+      const int c0 = w0 + (int)threadIdx.x;
       unsigned need = 0;
 #pragma unroll
       for (int j = 0; j < kStageWords; ++j)
@@ -798,7 +917,7 @@ __device__ __noinline__ int down_item(uint64_t kernarg, int q_arg, int state_arg
 #pragma unroll
         for (int j = 0; j < kStageWords; ++j) {
           const uint64_t* b = is_shared ? sgh + n : src;
-          w[j] = (cur >> j) & 1u ? load_agent(b + u0 + kThreads * j + threadIdx.x) : 0ull;
+          w[j] = (cur >> j) & 1u ? load_agent(b + w0 + kThreads * j + threadIdx.x) : 0ull;
         }
 #pragma unroll
         for (int j = 0; j < kStageWords; ++j) {
@@ -847,20 +966,21 @@ __device__ __noinline__ int down_item(uint64_t kernarg, int q_arg, int state_arg
   } else {
     // FP4 E8M0 at m >= 3: batches of 8 steps instead of 16 (measured at M=3:
     // 78.0 us against 78.8; at M=1 the 16-step batch is 0.2 us faster)
-    if (fmt == kFp4E8M0 && m >= 3) down_any<kFp4E8M0, true, 8>(ent, g_tile, m, i, p.d, r0, 0, i / 128, acc, stage);
+    if (fmt == kFp4E8M0 && p.m >= 3) down_any<kFp4E8M0, true, 8>(ent, g_tile, m, i, p.d, r0, 0, i / 128, acc, stage);
     else if (fmt == kFp4E8M0) down_any<kFp4E8M0, true>(ent, g_tile, m, i, p.d, r0, acc, stage);
     else if (fmt == kFp4F32) down_any<kFp4F32, true>(ent, g_tile, m, i, p.d, r0, acc, stage);
     else down_any<kBf16, true>(ent, g_tile, m, i, p.d, r0, acc, stage);
   }
   state = kShared ? 0 : 2 + s;
-  // lane (col = lane%16) holds rows 4*(lane/16)+c; column t (hi) + column m+t (lo)
-  // of token t are combined through the lane that owns column t.
-  uint64_t* part = p.part + (int64_t)s * m * p.d;
+  // lane (col = lane%16) holds rows 4*(lane/16)+c; column c (hi) + column m+c (lo)
+  // of a pair are combined through the lane that owns column c.
+  uint64_t* part = p.part + (int64_t)(kShared ? p.S : u0) * p.d;
   if (kShared && wave >= 2) return state;
-  // one routed slot and no shared expert: this item is its row group's only
-  // contributor and writes the rows itself (the value the row-group sum
-  // would give: 0 + the partial), with no round trip through the partials
-  const bool alone = !kShared && sh.n_routed == 1 && !p.shared;
+  // one routed slot, selected by every token, and no shared expert: this item
+  // is its row group's only contributor and writes the rows itself (the value
+  // the row-group sum would give: 0 + the partial; column c is token c), with
+  // no round trip through the partials
+  const bool alone = !kShared && lone_slot(p, sh);
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const int col = lane & 15;
@@ -895,29 +1015,29 @@ __device__ __noinline__ void down_finish(uint64_t kernarg, int q_arg) {
   down_slot_of(p, q, is_shared, s, g, h);
   const int n_routed = sh.n_routed;
   if (!is_shared && s >= n_routed) return;
-  if (n_routed == 1 && !p.shared) return;  // the down item wrote its rows itself
+  if (lone_slot(p, sh)) return;  // the down item wrote its rows itself
   int last = n_routed > 0 ? down_index(p, n_routed - 1, g) : -1;
   if (p.shared && p.sd0 + 2 * g + 1 > last) last = p.sd0 + 2 * g + 1;
   if (q != last) return;
   const unsigned tag = g_sh.tag;
   const int m = p.m;
-  const int64_t stride = (int64_t)m * p.d;  // between slots
+  static_assert(kDownRows == 64, "a wave adds one token's rows");
   for (int c0 = 0; c0 < kDownRows * m; c0 += kThreads) {
     const int c = c0 + (int)threadIdx.x;
     const bool mine = c < kDownRows * m;
-    const int t = mine ? c / kDownRows : 0, dd = g * kDownRows + (mine ? c - t * kDownRows : 0);
-    const uint32_t off = (uint32_t)(t * p.d + dd);
+    const int t = __builtin_amdgcn_readfirstlane(mine ? c / kDownRows : 0), dd = g * kDownRows + (c & (kDownRows - 1));
+    const int np = __builtin_amdgcn_readfirstlane(sh.ntp[t]);
     float v = 0.0f;
-    for (int s0 = 0; s0 < n_routed; s0 += 8) {
+    for (int j0 = 0; j0 < np; j0 += 8) {
       float pv[8];
-      poll_tagged<8>(p.part + (int64_t)s0 * stride, stride, off, mine ? n_routed - s0 : 0, tag, pv, p.ctl, kWaitPart);
+      poll_tagged_pairs(p.part + dd, sh.tpair[t] + j0, p.d, mine ? np - j0 : 0, tag, pv, p.ctl, kWaitPart);
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        if (s0 + j < n_routed) v = __fadd_rn(v, pv[j]);
+        if (j0 + j < np) v = __fadd_rn(v, pv[j]);
     }
     if (p.shared) {
       float pv[1];
-      poll_tagged<1>(p.part + (int64_t)p.S * stride, stride, off, mine ? 1 : 0, tag, pv, p.ctl, kWaitPart);
+      poll_tagged<1>(p.part + (int64_t)p.S * p.d, 0, (uint32_t)(t * p.d + dd), mine ? 1 : 0, tag, pv, p.ctl, kWaitPart);
       v = __fadd_rn(v, pv[0]);
     }
     if (mine) {
@@ -1250,10 +1370,10 @@ int launch_layer(const char* name, const void* x, int64_t m, int64_t d, int64_t 
   p.score_stride = (int)score_stride_words(m, n_experts);
   ws += scores_bytes(m, n_experts);
   p.act = (uint64_t*)ws;
-  p.sgh = p.act + (size_t)p.S * m * i;
+  p.sgh = p.act + (size_t)p.S * i;
   ws += act_bytes(m, i, top_k);
   p.part = (uint64_t*)ws;
-  p.fin = tail ? p.part + (size_t)(p.S + 1) * m * d : nullptr;
+  p.fin = tail ? p.part + (size_t)(p.S + m) * d : nullptr;
   p.wipe = (uint4*)((char*)workspace + kCtlBytes);
   p.wipe_n = (int64_t)((workspace_bytes - kCtlBytes) / 16);
   p.status_out = status_out;

@@ -318,3 +318,49 @@ def test_lone_slot_every_format(layer, dev, fmt):
     torch.cuda.synchronize()
     assert ops.moe_layer_status(dev) == 0
     assert torch.count_nonzero(z[1]) == 0 and torch.count_nonzero(z[0]) == 0
+
+
+@pytest.mark.parametrize("pattern", ["disjoint", "same", "mixed", "lone_of_some"])
+def test_routed_layer_pairs(layer, dev, pattern):
+    """The (slot, token) pairs a launch computes: 128 slots of one pair each,
+    16 slots of 8 pairs each, repeats and invalid ids with a token that
+    selects nothing, and one slot that not every token selects."""
+    store, _, _ = layer
+    m, k = 8, 16
+    idx = torch.arange(m * k, device=dev).reshape(m, k) * 2
+    if pattern == "same":
+        idx = torch.stack([torch.roll(torch.arange(k, device=dev) * 9, t) for t in range(m)])
+    elif pattern == "mixed":
+        idx[1] = torch.tensor([7, 7, -1, 300, 3, 9, 3, 7, 200, 11, 250, 4, 4, 4, 0, 255], device=dev)
+        idx[3] = idx[1].flip(0)
+        idx[5] = -1
+    elif pattern == "lone_of_some":
+        idx = torch.full((m, k), -1, dtype=torch.int64, device=dev)
+        idx[2, 5] = idx[6, 0] = 77
+    w = torch.rand(m, k, device=dev, generator=torch.Generator(dev).manual_seed(5)) + 0.1
+    x = synthetic.hidden(SEED, 40, m, D, dev)
+    for shared in (None, store.shared_entry(0)):
+        got = routed(x, idx, store.table(0), shared, w=w, k=k)
+        f32 = torch.empty(m, D, dtype=torch.float32, device=dev)
+        out, _ = ops.moe_decode(x, idx, w, store.table(0), ops.SCALE_E8M0, shared, 10.0, out_f32=f32, d=D, i=I)
+        torch.cuda.synchronize()
+        assert ops.moe_layer_status(dev) == 0
+        assert torch.equal(got[0], out) and torch.equal(got[1], f32)
+
+
+def test_expert_that_is_not_finite_reaches_only_its_tokens(layer, dev):
+    """A NaN scale byte makes every product of its expert NaN: the tokens that select it and no others."""
+    store, _, _ = layer
+    views = [t.clone() for t in store.expert_views(0, 5)]
+    for s in (views[1], views[5]):
+        s.view(torch.uint8)[:, 0] = 255
+    table = store.table(0).clone()
+    table[5] = torch.tensor([t.data_ptr() for t in views], dtype=torch.int64, device=dev)
+    idx = torch.tensor([[5, 9], [9, 12], [12, 5]], device=dev)
+    w = torch.full((3, 2), 0.5, device=dev)
+    x = synthetic.hidden(SEED, 41, 3, D, dev)
+    a = routed(x, idx, table, None, w=w, k=2)[1]
+    b = torch.empty_like(a)
+    ops.moe_decode(x, idx, w, table, ops.SCALE_E8M0, None, 10.0, out_f32=b, d=D, i=I)
+    for got in (a, b):
+        assert torch.isnan(got[[0, 2]]).all() and torch.isfinite(got[1]).all()
