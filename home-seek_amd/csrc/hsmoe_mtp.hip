@@ -10,9 +10,10 @@
 //  - 1 token, d <= 4096: one wave per vocab row, 1 KB per load instruction,
 //    the lane's hidden-state columns in fp64 registers, the row's partial
 //    sums added across the wave (lm_head_row_kernel);
-//  - 2..4 tokens: v_mfma_f64_4x4x4_4b_f64 over 4-row tiles, the bf16 hidden
+//  - 2..8 tokens: v_mfma_f64_4x4x4_4b_f64 over 4-row tiles, the bf16 hidden
 //    states in LDS (lm_head_mfma_kernel);
-//  - 1 token with d > 4096, or 5..8 tokens: one lane per vocab row summing in fp64 FMAs, the
+//  - 1 token with d > 4096, or hidden states that are not 16-byte aligned: one
+//    lane per vocab row summing in fp64 FMAs, the
 //    hidden states widened to fp64 on their way into LDS when they fit
 //    (n_tok * d * 8 <= kLdsHBytes), else widened into the workspace by
 //    widen_h_kernel and read from there (lm_head_kernel); the inner loop reads
@@ -31,7 +32,7 @@ constexpr int kMaxTok = 8;
 constexpr int kWaves = 8;
 constexpr int kRowsPerBlock = 64 * kWaves;
 constexpr size_t kLdsHBytes = 128 * 1024;  // hidden states in LDS up to this size (one workgroup per CU)
-constexpr int kMfmaMinTok = 2;  // the fp64 MFMA form serves 2..4 tokens (one token: the row-per-lane form)
+constexpr int kMfmaMinTok = 2;  // the fp64 MFMA form serves 2..8 tokens (one token: the row-per-wave form)
 
 struct Workspace {
   unsigned long long key[kMaxTok];
@@ -96,6 +97,11 @@ __device__ __forceinline__ double bf16_elem(const uint4& q, int e) {
   return (double)__uint_as_float((e & 1) ? (word & 0xffff0000u) : (word << 16));
 }
 
+// Rows per step: short rows two to eight at a time, so that a wave's loads in
+// flight stay at about 8 KB (d = 2048, one row per step: 4.5 TB/s).
+template <int kC>
+constexpr int row_step() { return kC >= 5 ? 1 : kC >= 3 ? 2 : kC == 2 ? 4 : 8; }
+
 template <int kC>
 __global__ void __launch_bounds__(64 * kRowWaves)
     lm_head_row_kernel(const uint16_t* __restrict__ w, const uint16_t* __restrict__ hb, int64_t vocab,
@@ -105,6 +111,7 @@ __global__ void __launch_bounds__(64 * kRowWaves)
   __shared__ int s_last;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   constexpr int kRowQ = 64 * kC;  // 16-byte chunks per row
+  constexpr int kR = row_step<kC>();
   double hv[kC][8];
 #pragma unroll
   for (int j = 0; j < kC; ++j) {
@@ -115,34 +122,51 @@ __global__ void __launch_bounds__(64 * kRowWaves)
   const uint4* __restrict__ wq = reinterpret_cast<const uint4*>(w) + lane;
   const int64_t nwv = (int64_t)gridDim.x * kRowWaves;
   unsigned long long key = 0;
-  auto load = [&](uint4 (&q)[kC], int64_t v) __attribute__((always_inline)) {
+  // step v: rows kR v .. kR v + kR - 1 (rows past the end read the last row; their sums are dropped)
+  auto load = [&](uint4 (&q)[kR][kC], int64_t v) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < kC; ++j) q[j] = wq[v * kRowQ + 64 * j];
+    for (int r = 0; r < kR; ++r) {
+      const int64_t row = kR * v + r < vocab ? kR * v + r : vocab - 1;
+#pragma unroll
+      for (int j = 0; j < kC; ++j) q[r][j] = wq[row * kRowQ + 64 * j];
+    }
   };
-  auto sum_row = [&](const uint4 (&q)[kC], int64_t v) __attribute__((always_inline)) {
-    double acc = 0.0;
+  auto sum_row = [&](const uint4 (&q)[kR][kC], int64_t v) __attribute__((always_inline)) {
+    double acc[kR];
 #pragma unroll
-    for (int j = 0; j < kC; ++j)
+    for (int r = 0; r < kR; ++r) {
+      acc[r] = 0.0;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc = __fma_rn(hv[j][e], bf16_elem(q[j], e), acc);
+      for (int j = 0; j < kC; ++j)
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 64);
-    const uint32_t bits = f64_to_bf16_bits(acc);
-    if (lane == 0 && logits) logits[v] = (uint16_t)bits;
-    const unsigned long long k1 = logit_key(bits, v);
-    key = k1 > key ? k1 : key;
+        for (int e = 0; e < 8; ++e) acc[r] = __fma_rn(hv[j][e], bf16_elem(q[r][j], e), acc[r]);
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1)
+#pragma unroll
+      for (int r = 0; r < kR; ++r) acc[r] += __shfl_xor(acc[r], off, 64);
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+      const int64_t row = kR * v + r;
+      if (row >= vocab) break;
+      const uint32_t bits = f64_to_bf16_bits(acc[r]);
+      if (lane == 0 && logits) logits[row] = (uint16_t)bits;
+      const unsigned long long k1 = logit_key(bits, row);
+      key = k1 > key ? k1 : key;
+    }
   };
+  const int64_t nsteps = (vocab + kR - 1) / kR;
   int64_t v = (int64_t)blockIdx.x * kRowWaves + wave;
-  uint4 qa[kC], qb[kC];
-  if (v < vocab) load(qa, v);
-  // two rows per turn: the row after next is loaded while this one is summed
-  while (v < vocab) {
+  uint4 qa[kR][kC], qb[kR][kC];
+  if (v < nsteps) load(qa, v);
+  // two steps per turn: the next step's rows are loaded while this one's are summed
+  while (v < nsteps) {
     const int64_t v1 = v + nwv;
-    if (v1 < vocab) load(qb, v1);
+    if (v1 < nsteps) load(qb, v1);
     sum_row(qa, v);
-    if (v1 >= vocab) break;
+    if (v1 >= nsteps) break;
     const int64_t v2 = v1 + nwv;
-    if (v2 < vocab) load(qa, v2);
+    if (v2 < nsteps) load(qa, v2);
     sum_row(qb, v1);
     v = v2;
   }
@@ -169,7 +193,7 @@ int launch_row(const uint16_t* w, const uint16_t* h, int64_t vocab, const int64_
   // against 179-180 with two per CU (320 or 384 workgroups, uneven over the
   // CUs: 185-205)
   const int64_t blocks = device_cus();
-  const int64_t need = (vocab + kRowWaves - 1) / kRowWaves;
+  const int64_t need = (vocab + kRowWaves * row_step<kC>() - 1) / (kRowWaves * row_step<kC>());
   const unsigned nb = (unsigned)(need < blocks ? need : blocks);
   hipLaunchKernelGGL((lm_head_row_kernel<kC>), dim3(nb), dim3(64 * kRowWaves), 0, st, w, h, vocab, ids, logits, pred,
                      result, ws);
@@ -177,7 +201,7 @@ int launch_row(const uint16_t* w, const uint16_t* h, int64_t vocab, const int64_
 }
 
 // ------------------------------------------------------------- fp64 MFMA form
-// For up to 4 tokens the dot products run on v_mfma_f64_4x4x4_4b_f64: four
+// For 2..8 tokens the dot products run on v_mfma_f64_4x4x4_4b_f64: four
 // blocks of D (4x4) += A (4x4) B (4x4) in fp64 per instruction, operands
 // (fitted on the device) A_b[i][k] in lane 16k + 4b + i, B_b[k][j] in lane
 // 16k + 4b + j, D_b[i][j] in lane 16i + 4b + j.  A wave works through tiles
@@ -196,14 +220,17 @@ int launch_row(const uint16_t* w, const uint16_t* h, int64_t vocab, const int64_
 // next group's loads go out while a group is multiplied (one group ahead:
 // 202 us at T = 3 over the 129,280 x 4096 head against 207 with four; the
 // same loads with no arithmetic run at 182-187).
-// The hidden states sit in LDS as bf16 [4][d]; a B lane reads the same
+// 5..8 tokens take a second instruction per A operand for columns 4..7, and
+// two tiles per step so that a hidden value is converted once per 8 rows:
+// bound by the conversions and the fp64 matrix rate, T = 5 over the 129,280 x
+// 4096 head 532 us (a row per lane, fp64 FMAs) -> 290 with one tile per step
+// -> 232 with two (four spill: 271).
+// The hidden states sit in LDS as bf16 [4 or 8][d]; a B lane reads the same
 // columns as its A lane in 16-byte LDS loads.  Products of bf16 values are
 // exact in fp64 and every partial sum is a subset sum of a row's products,
 // so a logit is the row's exact sum rounded once to bf16 whenever that sum is
 // exact in fp64, as for the row-per-lane form.
-constexpr int kMfmaWaves = 4;
 constexpr int kMfmaW = 4;                  // 16-byte loads per lane and group (8 k each)
-constexpr int kMfmaAhead = 1;             // groups in flight per wave (64 bytes per lane)
 constexpr int kMfmaGroupCols = 128 * kMfmaW;  // columns of a row per group
 constexpr int kMfmaResidentWaves = 4096;   // 256 CUs x 4 SIMDs x 4 waves
 
@@ -213,97 +240,132 @@ __device__ __forceinline__ double bf16_lane(const uint4& q, int n) {
 }
 
 template <int kTok>
-__global__ void __launch_bounds__(64 * kMfmaWaves)
+constexpr int mfma_waves() { return kTok > 4 ? 8 : 4; }  // waves per workgroup
+
+template <int kTok>
+constexpr int mfma_tiles() { return kTok > 4 ? 2 : 1; }  // 4-row tiles per wave step
+
+template <int kTok>
+__global__ void __launch_bounds__(64 * mfma_waves<kTok>(), 4)
     lm_head_mfma_kernel(const uint16_t* __restrict__ w, const uint16_t* __restrict__ h, int64_t d, int64_t vocab,
                         const int64_t* __restrict__ ids, uint16_t* __restrict__ logits,
                         int64_t* __restrict__ pred_out, int64_t* __restrict__ result_out,
                         Workspace* __restrict__ ws) {
-  extern __shared__ uint16_t s_hb[];  // [4][d] bf16, rows >= kTok zero
-  __shared__ unsigned long long s_key[kMfmaWaves][4];
+  constexpr int kMfmaWaves = mfma_waves<kTok>();
+  constexpr int kG = (kTok + 3) / 4;  // groups of 4 token columns
+  extern __shared__ uint16_t s_hb[];  // [4 kG][d] bf16, rows >= kTok zero
+  __shared__ unsigned long long s_key[kMfmaWaves][4 * kG];
   __shared__ int s_last;
   const int chunks = (int)(d / 8);
-  for (int c = threadIdx.x; c < 4 * chunks; c += 64 * kMfmaWaves) {
+  for (int c = threadIdx.x; c < 4 * kG * chunks; c += 64 * kMfmaWaves) {
     const int t = c / chunks;
     reinterpret_cast<uint4*>(s_hb)[c] = t < kTok ? reinterpret_cast<const uint4*>(h)[c] : make_uint4(0, 0, 0, 0);
   }
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int lo = lane & 3, slot = lane >> 2;  // A row i / B token j; (block, k) pair
-  const int64_t ntile = (vocab + 3) / 4;
-  // tiles t0, t0 + nwv, t0 + 2 nwv, ...: at any moment the grid streams one contiguous window of the head
+  constexpr int kR = mfma_tiles<kTok>();  // 4-row tiles per wave step
+  const int64_t ntile = (vocab + 4 * kR - 1) / (4 * kR);
+  // steps t0, t0 + nwv, t0 + 2 nwv, ...: at any moment the grid streams one contiguous window of the head
   const int64_t t0 = (int64_t)blockIdx.x * kMfmaWaves + wave, nwv = (int64_t)gridDim.x * kMfmaWaves;
   const int64_t ntw = t0 < ntile ? (ntile - 1 - t0) / nwv + 1 : 0;
   const int ng = (int)(d / kMfmaGroupCols);
-  const int64_t nf = ntw * ng;  // (tile, group) steps of this wave
+  const int64_t nf = ntw * ng;  // (step, group) loads of this wave
   const uint4* hq = reinterpret_cast<const uint4*>(s_hb + (int64_t)lo * d + 8 * slot);
-  auto row_ptr = [&](int64_t t) {  // rows past the end read the last row; their sums are dropped
-    const int64_t r = 4 * t + lo < vocab ? 4 * t + lo : vocab - 1;
-    return reinterpret_cast<const uint4*>(w + r * d + 8 * slot);
-  };
-  unsigned long long key = 0;
-  uint4 q[kMfmaAhead][kMfmaW];
-  int64_t lt = t0;  // tile and group of the next load
-  int lg = 0;
-  const uint4* lp = row_ptr(lt);
+  const uint4* lp[kR];
+  auto set_rows = [&](int64_t t) __attribute__((always_inline)) {  // rows past the end read the last row; their sums are dropped
 #pragma unroll
-  for (int p = 0; p < kMfmaAhead; ++p) {
-#pragma unroll
-    for (int h2 = 0; h2 < kMfmaW; ++h2) q[p][h2] = p < nf ? lp[16 * (kMfmaW * lg + h2)] : make_uint4(0, 0, 0, 0);
-    if (p < nf && ++lg == ng) {
-      lg = 0;
-      lp = row_ptr(lt += nwv);
+    for (int r = 0; r < kR; ++r) {
+      const int64_t v = 4 * (kR * t + r) + lo < vocab ? 4 * (kR * t + r) + lo : vocab - 1;
+      lp[r] = reinterpret_cast<const uint4*>(w + v * d + 8 * slot);
     }
-  }
-  double acc0 = 0.0, acc1 = 0.0;
+  };
+  unsigned long long key[kG] = {};
+  uint4 q[kR][kMfmaW];
+  int64_t lt = t0;  // step and group of the next load
+  int lg = 0;
+  set_rows(lt);
+  auto advance = [&]() __attribute__((always_inline)) {
+    if (++lg == ng) {
+      lg = 0;
+      set_rows(lt += nwv);
+    }
+  };
+#pragma unroll
+  for (int r = 0; r < kR; ++r)
+#pragma unroll
+    for (int h2 = 0; h2 < kMfmaW; ++h2) q[r][h2] = nf > 0 ? lp[r][16 * h2] : make_uint4(0, 0, 0, 0);
+  if (nf > 0) advance();
+  double acc0[kR][kG] = {}, acc1[kR][kG] = {};
   int cg = 0;  // group of the step being summed
   int64_t ct = t0;
-  for (int64_t f0 = 0; f0 < nf; f0 += kMfmaAhead) {
+  for (int64_t f = 0; f < nf; ++f) {
+    const bool more = f + 1 < nf;
 #pragma unroll
-    for (int p = 0; p < kMfmaAhead; ++p) {
-      if (f0 + p < nf) {
-        const bool more = f0 + p + kMfmaAhead < nf;
+    for (int h2 = 0; h2 < kMfmaW; ++h2) {
+      uint4 cur[kR], hv[kG];
 #pragma unroll
-        for (int h2 = 0; h2 < kMfmaW; ++h2) {
-          const uint4 cur = q[p][h2];
-          if (more) q[p][h2] = lp[16 * (kMfmaW * lg + h2)];
-          const uint4 hv = hq[16 * (kMfmaW * cg + h2)];
+      for (int r = 0; r < kR; ++r) {
+        cur[r] = q[r][h2];
+        if (more) q[r][h2] = lp[r][16 * (kMfmaW * lg + h2)];
+      }
 #pragma unroll
-          for (int n = 0; n < 8; n += 2) {
-            acc0 = __builtin_amdgcn_mfma_f64_4x4x4f64(bf16_lane(cur, n), bf16_lane(hv, n), acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f64_4x4x4f64(bf16_lane(cur, n + 1), bf16_lane(hv, n + 1), acc1, 0, 0, 0);
-          }
+      for (int tg = 0; tg < kG; ++tg) hv[tg] = hq[(int64_t)tg * (d / 2) + 16 * (kMfmaW * cg + h2)];
+#pragma unroll
+      for (int n = 0; n < 8; n += 2) {
+        double h0[kG], h1[kG];
+#pragma unroll
+        for (int tg = 0; tg < kG; ++tg) {
+          h0[tg] = bf16_lane(hv[tg], n);
+          h1[tg] = bf16_lane(hv[tg], n + 1);
         }
-        if (more && ++lg == ng) {
-          lg = 0;
-          lp = row_ptr(lt += nwv);
-        }
-        if (++cg == ng) {
-          // lane (i, b, j): block b's partial of row 4 ct + i, token j; add the 4 blocks
-          double s = acc0 + acc1;
-          s = s + __shfl_xor(s, 4, 64);
-          s = s + __shfl_xor(s, 8, 64);
-          const int64_t v = 4 * ct + (lane >> 4);
-          if ((lane & 12) == 0 && lo < kTok && v < vocab) {
-            const uint32_t bits = f64_to_bf16_bits(s);
-            if (logits) logits[lo * vocab + v] = (uint16_t)bits;
-            const unsigned long long k1 = logit_key(bits, v);
-            key = k1 > key ? k1 : key;
+#pragma unroll
+        for (int r = 0; r < kR; ++r) {
+          const double w0 = bf16_lane(cur[r], n), w1 = bf16_lane(cur[r], n + 1);
+#pragma unroll
+          for (int tg = 0; tg < kG; ++tg) {
+            acc0[r][tg] = __builtin_amdgcn_mfma_f64_4x4x4f64(w0, h0[tg], acc0[r][tg], 0, 0, 0);
+            acc1[r][tg] = __builtin_amdgcn_mfma_f64_4x4x4f64(w1, h1[tg], acc1[r][tg], 0, 0, 0);
           }
-          acc0 = 0.0;
-          acc1 = 0.0;
-          cg = 0;
-          ct += nwv;
         }
       }
     }
-  }
-  // the wave's best key of token j: lanes with equal lane & 3
+    if (more) advance();
+    if (++cg == ng) {
+      // lane (i, b, j): block b's partial of row i of the tile, token 4 tg + j; add the 4 blocks
 #pragma unroll
-  for (int off = 4; off < 64; off <<= 1) {
-    const unsigned long long o = __shfl_xor(key, off, 64);
-    key = o > key ? o : key;
+      for (int r = 0; r < kR; ++r) {
+        const int64_t v = 4 * (kR * ct + r) + (lane >> 4);
+#pragma unroll
+        for (int tg = 0; tg < kG; ++tg) {
+          double s = acc0[r][tg] + acc1[r][tg];
+          s = s + __shfl_xor(s, 4, 64);
+          s = s + __shfl_xor(s, 8, 64);
+          const int t = 4 * tg + lo;
+          if ((lane & 12) == 0 && t < kTok && v < vocab) {
+            const uint32_t bits = f64_to_bf16_bits(s);
+            if (logits) logits[t * vocab + v] = (uint16_t)bits;
+            const unsigned long long k1 = logit_key(bits, v);
+            key[tg] = k1 > key[tg] ? k1 : key[tg];
+          }
+          acc0[r][tg] = 0.0;
+          acc1[r][tg] = 0.0;
+        }
+      }
+      cg = 0;
+      ct += nwv;
+    }
   }
-  if (lane < 4) s_key[wave][lane] = key;
+  // the wave's best key of token 4 tg + j: lanes with equal lane & 3
+#pragma unroll
+  for (int tg = 0; tg < kG; ++tg) {
+#pragma unroll
+    for (int off = 4; off < 64; off <<= 1) {
+      const unsigned long long o = __shfl_xor(key[tg], off, 64);
+      key[tg] = o > key[tg] ? o : key[tg];
+    }
+    if (lane < 4) s_key[wave][4 * tg + lane] = key[tg];
+  }
   __syncthreads();
   if (threadIdx.x < kTok) {
     unsigned long long k = 0;
@@ -323,11 +385,12 @@ template <int kTok>
 int launch_mfma(const uint16_t* w, const uint16_t* h, int64_t d, int64_t vocab, const int64_t* ids, uint16_t* logits,
                 int64_t* pred, int64_t* result, Workspace* ws, hipStream_t st) {
   // every wave resident at once (no more waves than tiles)
-  const int64_t ntile = (vocab + 3) / 4;
+  const int64_t ntile = (vocab + 4 * mfma_tiles<kTok>() - 1) / (4 * mfma_tiles<kTok>());
   const int64_t nw = ntile < kMfmaResidentWaves ? ntile : kMfmaResidentWaves;
+  constexpr int kMfmaWaves = mfma_waves<kTok>(), kRowsH = (kTok + 3) / 4 * 4;
   const unsigned nb = (unsigned)((nw + kMfmaWaves - 1) / kMfmaWaves);
-  const size_t lds = (size_t)4 * (size_t)d * 2;
-  constexpr size_t kMaxLds = (size_t)4 * 8192 * 2;  // d <= 8192: 64 KiB of hidden states, beyond the default
+  const size_t lds = (size_t)kRowsH * (size_t)d * 2;
+  constexpr size_t kMaxLds = (size_t)kRowsH * 8192 * 2;  // d <= 8192: 64 or 128 KiB, beyond the default
   static bool raised = false;                       // allow it once per instantiation
   if (!raised) {
     if (hipFuncSetAttribute((const void*)lm_head_mfma_kernel<kTok>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -487,13 +550,16 @@ extern "C" int hsmoe_lm_head_accept(const void* h, const void* lm_head, int64_t 
   Workspace* ws = (Workspace*)workspace;
   const uint16_t* w = (const uint16_t*)lm_head;
   uint16_t* lg = (uint16_t*)logits_out;
-  if (n_tok >= kMfmaMinTok && n_tok <= 4 && aligned(h, 16)) {
+  if (n_tok >= kMfmaMinTok && aligned(h, 16)) {
     const uint16_t* hb = (const uint16_t*)h;
     switch (n_tok) {
-      case 1: return launch_mfma<1>(w, hb, d, vocab, ids, lg, pred_out, result_out, ws, st);
       case 2: return launch_mfma<2>(w, hb, d, vocab, ids, lg, pred_out, result_out, ws, st);
       case 3: return launch_mfma<3>(w, hb, d, vocab, ids, lg, pred_out, result_out, ws, st);
-      default: return launch_mfma<4>(w, hb, d, vocab, ids, lg, pred_out, result_out, ws, st);
+      case 4: return launch_mfma<4>(w, hb, d, vocab, ids, lg, pred_out, result_out, ws, st);
+      case 5: return launch_mfma<5>(w, hb, d, vocab, ids, lg, pred_out, result_out, ws, st);
+      case 6: return launch_mfma<6>(w, hb, d, vocab, ids, lg, pred_out, result_out, ws, st);
+      case 7: return launch_mfma<7>(w, hb, d, vocab, ids, lg, pred_out, result_out, ws, st);
+      default: return launch_mfma<8>(w, hb, d, vocab, ids, lg, pred_out, result_out, ws, st);
     }
   }
   if (n_tok == 1 && d <= 4096 && aligned(h, 16)) {  // one token: row per wave (d > 4096: row per lane)

@@ -138,6 +138,23 @@ def test_lm_head_logits_argmax_bit_exact(dev, n_tok, vocab, d):
     assert result.cpu().tolist() == [n, bonus]
 
 
+# 5..8 tokens: 8-row steps with a ragged end, fewer steps than waves, the largest hidden size (128 KiB of LDS);
+# one token with short rows, several rows per step: ragged ends, fewer rows than a step
+@pytest.mark.parametrize("n_tok,vocab,d", [(5, 40003, 4096), (7, 9, 512), (8, 1001, 8192), (6, 2050, 1536),
+                                           (1, 4099, 1024), (1, 5, 512), (1, 20001, 2048), (1, 3, 1024), (1, 7, 1536)])
+def test_lm_head_row_steps_bit_exact(dev, n_tok, vocab, d):
+    h = synthetic.hidden(n_tok, 1, n_tok, d, dev)
+    lm = synthetic.normal_bf16(n_tok, 77, (vocab, d), 0.0, 0.02, dev)
+    ids = torch.arange(n_tok, device=dev)
+    ref = orc.logits_bf16(orc.to_np_bf16(h), orc.to_np_bf16(lm))
+    shifted = torch.empty(h.numel() + 4, dtype=torch.bfloat16, device=dev)[4:].view_as(h).copy_(h)
+    for hh in (h, shifted):  # the second is not 16-byte aligned: the row-per-lane form
+        for _ in range(2):
+            logits, pred, _ = ops.lm_head_accept(hh, lm, ids)
+            assert np.array_equal(orc.to_np_bf16(logits), ref)
+            assert np.array_equal(pred.cpu().numpy(), orc.bf16_to_f32(ref).argmax(axis=1))
+
+
 def test_lm_head_accept_kats_on_device(dev):
     """The reference's accept/reject KATs (tests/test_mtp.py:355-456) with one-hot lm_head rows."""
     d, vocab = 512, 128
