@@ -21,8 +21,7 @@
 //            shared expert's M pairs.  Each bucket is cut into gate/up chunks
 //            (<= 32 pairs, or <= 64 for a bucket of more than 32, those first)
 //            and into down chunks of <= 32 pairs.
-//   gate_up  grid (chunk, 64-row block of I), one launch for the routed
-//            experts and one for the shared expert: wave w takes rows
+//   gate_up  grid (chunk, 64-row block of I): wave w takes rows
 //            +16w..+16 of W1 and W3 over all of D in K-chunks of 256 columns.
 //            While chunk kc is multiplied, the token tile of kc+1 is in flight
 //            to registers (then LDS) and the weights of kc+2 to a third
@@ -45,6 +44,7 @@ namespace hsmoe {
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kGroupThreads = 1024;  // group kernel: one workgroup per expert and CU
 constexpr int kChunk = 32;        // tokens per chunk (two 16-token MFMA tiles)
 constexpr int kBigChunk = 64;     // tokens per chunk of an expert with more than kChunk pairs
 constexpr int kGuRT = 1;          // 16-row tiles per wave, gate/up (W1 and W3)
@@ -57,9 +57,8 @@ constexpr int kMaxPairs = 12288;  // m * top_k per call (LDS of the group kernel
 constexpr int kMaxExperts = 1024;
 
 struct Header {
-  int n_routed_chunks;  // gate/up chunks of routed experts (big experts' first); the shared expert's follow
-  int n_pairs;
-  int n_dn_chunks;      // down chunks of routed experts (kChunk pairs each); the shared expert's follow
+  int n_gu;  // gate/up chunks: the shared expert's, then the routed experts' (big ones' first)
+  int n_dn;  // down chunks: the shared expert's, then the routed experts'
 };
 
 struct PrefillParams {
@@ -85,7 +84,7 @@ struct PrefillParams {
   uint16_t* out_bf16;      // [m, d] or null
   int n_experts;
   int m, d, i, top_k;
-  int scale_fmt;  // kFp4E8M0 or kFp4F32 for routed FP4 experts
+  int n_sh_gu, n_sh_dn;  // chunks of the shared expert's m pairs in either list
   float limit;
 };
 
@@ -98,6 +97,7 @@ struct PrefillParams {
 __device__ __forceinline__ int chunk_size(int cnt) { return cnt > kChunk ? kBigChunk : kChunk; }
 
 // Sum over the block of v (every thread passes its own value).
+template <int kWaves>
 __device__ __forceinline__ int block_sum(int v, int* s_red) {
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
@@ -106,7 +106,7 @@ __device__ __forceinline__ int block_sum(int v, int* s_red) {
   __syncthreads();
   int t = 0;
 #pragma unroll
-  for (int w = 0; w < kThreads / 64; ++w) t += s_red[w];
+  for (int w = 0; w < kWaves; ++w) t += s_red[w];
   return t;
 }
 
@@ -114,67 +114,75 @@ __device__ __forceinline__ int block_sum(int v, int* s_red) {
 // writes the header, the shared expert's pairs and the slots of invalid ids.
 // Every workgroup histograms the whole pair list in LDS, so the offsets of
 // expert e (pairs and chunks of the experts before it) need no second pass.
-// Within an expert, pairs keep (t, j) order: blocks of 256 pairs in order,
-// ranked by wave ballots.
-__global__ void __launch_bounds__(kThreads) prefill_group_kernel(PrefillParams p) {
-  __shared__ int s_e[kMaxPairs];
+// Within an expert, pairs keep (t, j) order: each wave counts, then places, the
+// hits of its contiguous share of the list, ranked by ballots.  The shared
+// expert's chunks come first in both lists: every token is in one of them, so
+// its workgroups are the fullest, and they run under the routed stream (as
+// launches of their own they took 25 MB of weights 60 + 40 us at m = 509).
+__global__ void __launch_bounds__(kGroupThreads) prefill_group_kernel(PrefillParams p) {
+  constexpr int kWaves = kGroupThreads / 64;
+  __shared__ uint16_t s_e[kMaxPairs];  // expert of pair q, kNone: invalid id or absent expert
   __shared__ int s_cnt[kMaxExperts];
   __shared__ bool s_ok[kMaxExperts];  // expert e has a table entry
-  __shared__ int s_red[kThreads / 64];
-  __shared__ int s_wc[kThreads / 64];
+  __shared__ int s_red[kWaves];
+  __shared__ int s_wc[kWaves];
+  constexpr int kNone = 0xffff;
   const int E = p.n_experts, K = p.top_k, P = p.m * K, me = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // which experts have a table entry: one load per expert, not one per pair
-  for (int e = threadIdx.x; e < E; e += kThreads) {
+  for (int e = threadIdx.x; e < E; e += kGroupThreads) {
     s_cnt[e] = 0;
     s_ok[e] = p.table[(int64_t)e * 6] != 0;
   }
   __syncthreads();
   // the pair ids, kIdBatch loads of a thread in flight at once
   constexpr int kIdBatch = 8;
-  for (int q0 = threadIdx.x; q0 < P; q0 += kIdBatch * kThreads) {
+  for (int q0 = threadIdx.x; q0 < P; q0 += kIdBatch * kGroupThreads) {
     int64_t ev[kIdBatch];
 #pragma unroll
-    for (int j = 0; j < kIdBatch; ++j) ev[j] = q0 + j * kThreads < P ? p.idx[q0 + j * kThreads] : -1;
+    for (int j = 0; j < kIdBatch; ++j) ev[j] = q0 + j * kGroupThreads < P ? p.idx[q0 + j * kGroupThreads] : -1;
 #pragma unroll
     for (int j = 0; j < kIdBatch; ++j) {
-      const int q = q0 + j * kThreads;
+      const int q = q0 + j * kGroupThreads;
       if (q >= P) break;
       const int64_t e = ev[j];
       const bool ok = e >= 0 && e < E && s_ok[e];
-      s_e[q] = ok ? (int)e : -1;
+      s_e[q] = (uint16_t)(ok ? (int)e : kNone);
       if (ok) atomicAdd(&s_cnt[e], 1);
     }
   }
   __syncthreads();
   if (me == E) {
     int pairs = 0, chunks = 0, dchunks = 0;
-    for (int e = threadIdx.x; e < E; e += kThreads) {
+    for (int e = threadIdx.x; e < E; e += kGroupThreads) {
       pairs += s_cnt[e];
       chunks += (s_cnt[e] + chunk_size(s_cnt[e]) - 1) / chunk_size(s_cnt[e]);
       dchunks += (s_cnt[e] + kChunk - 1) / kChunk;
     }
-    pairs = block_sum(pairs, s_red);
-    chunks = block_sum(chunks, s_red);
-    dchunks = block_sum(dchunks, s_red);
+    pairs = block_sum<kWaves>(pairs, s_red);
+    chunks = block_sum<kWaves>(chunks, s_red);
+    dchunks = block_sum<kWaves>(dchunks, s_red);
     if (threadIdx.x == 0) {
-      p.hdr->n_pairs = pairs + (p.shared ? p.m : 0);
-      p.hdr->n_routed_chunks = chunks;
-      p.hdr->n_dn_chunks = dchunks;
+      p.hdr->n_gu = p.n_sh_gu + chunks;
+      p.hdr->n_dn = p.n_sh_dn + dchunks;
     }
-    for (int q = threadIdx.x; q < P; q += kThreads)
-      if (s_e[q] < 0) p.pidx[(q / K) * (K + 1) + q % K] = -1;
-    for (int t = threadIdx.x; t < p.m; t += kThreads) {
+    for (int q = threadIdx.x; q < P; q += kGroupThreads)
+      if (s_e[q] == kNone) p.pidx[(q / K) * (K + 1) + q % K] = -1;
+    for (int t = threadIdx.x; t < p.m; t += kGroupThreads) {
       const int pos = pairs + t;
       p.pidx[t * (K + 1) + K] = p.shared ? pos : -1;
       if (!p.shared) continue;
       p.pair_tok[pos] = t;
       p.pair_w[pos] = 1.0f;
+      if (t % kBigChunk == 0) {
+        p.chunk_e[t / kBigChunk] = E;
+        p.chunk_p0[t / kBigChunk] = pos;
+        p.chunk_n[t / kBigChunk] = min(kBigChunk, p.m - t);
+      }
       if (t % kChunk == 0) {
-        const int ch = chunks + t / kChunk, dch = dchunks + t / kChunk;
-        p.chunk_e[ch] = p.dn_e[dch] = E;
-        p.chunk_p0[ch] = p.dn_p0[dch] = pos;
-        p.chunk_n[ch] = p.dn_n[dch] = min(kChunk, p.m - t);
+        p.dn_e[t / kChunk] = E;
+        p.dn_p0[t / kChunk] = pos;
+        p.dn_n[t / kChunk] = min(kChunk, p.m - t);
       }
     }
     return;
@@ -184,45 +192,45 @@ __global__ void __launch_bounds__(kThreads) prefill_group_kernel(PrefillParams p
   // chunks: the big experts' (expert order), then one per small expert (expert order)
   const bool big = cnt > kChunk;
   int off = 0, choff = 0, dnoff = 0;
-  for (int e = threadIdx.x; e < E; e += kThreads) {
+  for (int e = threadIdx.x; e < E; e += kGroupThreads) {
     const int c = s_cnt[e];
     if (e < me) off += c;
     if (e < me) dnoff += (c + kChunk - 1) / kChunk;
     if (c > kChunk && (!big || e < me)) choff += (c + kBigChunk - 1) / kBigChunk;  // every big expert's chunks first
     else if (!big && e < me && c > 0) ++choff;
   }
-  off = block_sum(off, s_red);
-  choff = block_sum(choff, s_red);
-  dnoff = block_sum(dnoff, s_red);
+  off = block_sum<kWaves>(off, s_red);
+  choff = p.n_sh_gu + block_sum<kWaves>(choff, s_red);
+  dnoff = p.n_sh_dn + block_sum<kWaves>(dnoff, s_red);
   const int cs = chunk_size(cnt);
+  // this wave's share of the list: its hits, then their places
+  const int per = (P + 64 * kWaves - 1) / (64 * kWaves) * 64;
+  const int q_lo = min(wave * per, P), q_hi = min(q_lo + per, P);
+  int hits = 0;
+  for (int q0 = q_lo; q0 < q_hi; q0 += 64)
+    hits += __popcll(__ballot(q0 + lane < q_hi && s_e[min(q0 + lane, P - 1)] == me));
+  if (lane == 0) s_wc[wave] = hits;
+  __syncthreads();
   int base = off;
-  for (int q0 = 0; q0 < P; q0 += kThreads) {
-    const int q = q0 + threadIdx.x;
-    const bool hit = q < P && s_e[q] == me;
+  for (int w = 0; w < wave; ++w) base += s_wc[w];
+  for (int q0 = q_lo; q0 < q_hi; q0 += 64) {
+    const int q = q0 + lane;
+    const bool hit = q < q_hi && s_e[min(q, P - 1)] == me;
     const unsigned long long bal = __ballot(hit);
-    if (lane == 0) s_wc[wave] = __popcll(bal);
-    __syncthreads();
-    int before = 0, total = 0;
-#pragma unroll
-    for (int w = 0; w < kThreads / 64; ++w) {
-      before += w < wave ? s_wc[w] : 0;
-      total += s_wc[w];
-    }
     if (hit) {
-      const int pos = base + before + __popcll(bal & ((1ull << lane) - 1ull));
+      const int pos = base + __popcll(bal & ((1ull << lane) - 1ull));
       p.pair_tok[pos] = q / K;
       p.pair_w[pos] = p.wts[q];
       p.pidx[(q / K) * (K + 1) + q % K] = pos;
     }
-    base += total;
-    __syncthreads();
+    base += __popcll(bal);
   }
-  for (int c = threadIdx.x; c * cs < cnt; c += kThreads) {
+  for (int c = threadIdx.x; c * cs < cnt; c += kGroupThreads) {
     p.chunk_e[choff + c] = me;
     p.chunk_p0[choff + c] = off + c * cs;
     p.chunk_n[choff + c] = min(cs, cnt - c * cs);
   }
-  for (int c = threadIdx.x; c * kChunk < cnt; c += kThreads) {
+  for (int c = threadIdx.x; c * kChunk < cnt; c += kGroupThreads) {
     p.dn_e[dnoff + c] = me;
     p.dn_p0[dnoff + c] = off + c * kChunk;
     p.dn_n[dnoff + c] = min(kChunk, cnt - c * kChunk);
@@ -237,24 +245,19 @@ __device__ __forceinline__ bf16x8 tile_frag(const uint16_t* t, int cols, int til
 
 struct Chunk {
   int e, p0, n;
+  bool shared;
   const uint64_t* ent;
 };
 
-// Chunk q of the routed experts (kShared = false) or of the shared expert,
-// from the gate/up list or (kDown) the down list.
-template <bool kShared, bool kDown>
+// Chunk q of the gate/up list or (kDown) the down list.
+template <bool kDown>
 __device__ __forceinline__ bool load_chunk(const PrefillParams& p, int q, Chunk& ch) {
-  const int nr = kDown ? p.hdr->n_dn_chunks : p.hdr->n_routed_chunks;
-  if (kShared) {
-    if (q * kChunk >= p.m) return false;
-    q += nr;
-  } else if (q >= nr) {
-    return false;
-  }
+  if (q >= (kDown ? p.hdr->n_dn : p.hdr->n_gu)) return false;
   ch.e = kDown ? p.dn_e[q] : p.chunk_e[q];
   ch.p0 = kDown ? p.dn_p0[q] : p.chunk_p0[q];
   ch.n = kDown ? p.dn_n[q] : p.chunk_n[q];
-  ch.ent = kShared ? p.shared : p.table + (int64_t)ch.e * 6;
+  ch.shared = ch.e == p.n_experts;
+  ch.ent = ch.shared ? p.shared : p.table + (int64_t)ch.e * 6;
   return true;
 }
 
@@ -497,40 +500,39 @@ __device__ void gate_up_chunk(const PrefillParams& p, const Chunk& ch, int r0, u
   }
 }
 
-// F: format of the chunks' weights (routed FP4 of the call's scale kind, or
-// the shared expert's FP8); table entries without scales take the bf16 path.
-template <int F, bool kShared>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(F == kFp8Block ? 2 : 4)))
+// F: format of the routed FP4 experts of the call's scale kind; the shared
+// expert's chunks are FP8; entries without scales (of either) take the bf16 path.
+template <int F>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
 prefill_gate_up_kernel(PrefillParams p) {
   __shared__ __align__(16) uint16_t xs[kBigChunk * (kCols + kPad)];
   __shared__ int s_tok[kBigChunk];
   const int nrb = p.i / kGuRows;
   Chunk ch;
-  if (!load_chunk<kShared, false>(p, blockIdx.x / nrb, ch)) return;
+  if (!load_chunk<false>(p, blockIdx.x / nrb, ch)) return;
   if (threadIdx.x < kBigChunk) s_tok[threadIdx.x] = threadIdx.x < ch.n ? p.pair_tok[ch.p0 + threadIdx.x] : 0;
   __syncthreads();
   const int r0 = (blockIdx.x % nrb) * kGuRows + 16 * kGuRT * (threadIdx.x >> 6);
   // routed E8M0 chunks read their scales through a per-lane cache (same weights)
   constexpr int FG = F == kFp4E8M0 ? kFp4E8M0Split : F;
-  if (!kShared && ch.n > kChunk && ch.ent[1]) {  // a big expert's chunk (the shared expert's hold at most kChunk)
-    gate_up_chunk<FG, kBigChunk, 1>(p, ch, r0, xs, s_tok);
-  } else if (ch.n > kChunk) {  // bf16 weights: the chunk as two kChunk halves (registers)
+  if (!ch.ent[1] || ch.shared) {  // bf16 or FP8 weights: a chunk of more than kChunk pairs as two halves (registers)
     for (int h0 = 0; h0 < ch.n; h0 += kChunk) {
       Chunk sub = ch;
       sub.p0 = ch.p0 + h0;
       sub.n = min(kChunk, ch.n - h0);
-      gate_up_chunk<kBf16, kChunk, 3>(p, sub, r0, xs, s_tok + h0);
+      if (ch.ent[1]) gate_up_chunk<kFp8Block, kChunk, 1>(p, sub, r0, xs, s_tok + h0);
+      else gate_up_chunk<kBf16, kChunk, 1>(p, sub, r0, xs, s_tok + h0);
     }
-  } else if (ch.ent[1]) {
-    gate_up_chunk<FG, kChunk, 3>(p, ch, r0, xs, s_tok);
+  } else if (ch.n > kChunk) {
+    gate_up_chunk<FG, kBigChunk, 1>(p, ch, r0, xs, s_tok);
   } else {
-    gate_up_chunk<kBf16, kChunk, 3>(p, ch, r0, xs, s_tok);
+    gate_up_chunk<FG, kChunk, 3>(p, ch, r0, xs, s_tok);
   }
 }
 
 // ---------------------------------------------------------------- down
 // F = kFp4E8M0Split: W2's E8M0 scales through a ScaleCache per row tile.
-template <int F>
+template <int F, int kBufs>
 __device__ void down_chunk(const PrefillParams& p, const Chunk& ch, int r0, uint16_t* as) {
   using W = WBuf<F, 1, kDnRT>;
   constexpr bool kSplit = F == kFp4E8M0Split;
@@ -549,7 +551,7 @@ __device__ void down_chunk(const PrefillParams& p, const Chunk& ch, int r0, uint
   }
   int kc = 0;
   auto src = [&](int pl, int tt) { return (pl ? p.act_lo : p.act_hi) + (int64_t)(ch.p0 + tt) * p.i; };
-  pipeline<F, 1, kDnRT, 2, kChunk, 3>(ch.ent, 4, p.d, r0 + r, p.i, g, ch.n, as, src, [&](const W& w) {
+  pipeline<F, 1, kDnRT, 2, kChunk, kBufs>(ch.ent, 4, p.d, r0 + r, p.i, g, ch.n, as, src, [&](const W& w) {
     if constexpr (kSplit) {
       if (kc > 0 && (kc & (ScaleCache::kSteps / 2 - 1)) == 0) {  // the next kSteps steps' scales
 #pragma unroll
@@ -593,16 +595,17 @@ __device__ void down_chunk(const PrefillParams& p, const Chunk& ch, int r0, uint
   }
 }
 
-template <int F, bool kShared>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(F == kFp8Block ? 2 : 3)))
+template <int F>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3)))
 prefill_down_kernel(PrefillParams p) {
   __shared__ __align__(16) uint16_t as[2 * kChunk * (kCols + kPad)];  // hi plane, lo plane
   const int nrb = p.d / kDnRows;
   Chunk ch;
-  if (!load_chunk<kShared, true>(p, blockIdx.x / nrb, ch)) return;
+  if (!load_chunk<true>(p, blockIdx.x / nrb, ch)) return;
   const int r0 = (blockIdx.x % nrb) * kDnRows + 16 * kDnRT * (threadIdx.x >> 6);
-  if (ch.ent[1]) down_chunk<F == kFp4E8M0 ? kFp4E8M0Split : F>(p, ch, r0, as);  // routed E8M0: cached scales
-  else down_chunk<kBf16>(p, ch, r0, as);
+  if (!ch.ent[1]) down_chunk<kBf16, 1>(p, ch, r0, as);
+  else if (ch.shared) down_chunk<kFp8Block, 1>(p, ch, r0, as);
+  else down_chunk<F == kFp4E8M0 ? kFp4E8M0Split : F, 3>(p, ch, r0, as);  // routed E8M0: cached scales
 }
 
 // ---------------------------------------------------------------- combine
@@ -741,28 +744,22 @@ extern "C" int hsmoe_moe_prefill(const void* x, int64_t m, int64_t d, int64_t i,
   p.d = (int)d;
   p.i = (int)i;
   p.top_k = top_k;
-  p.scale_fmt = scale_kind == HSMOE_SCALE_E8M0 ? kFp4E8M0 : kFp4F32;
   p.limit = swiglu_limit;
   hipStream_t st = (hipStream_t)stream;
-  const int64_t C = max_routed_chunks(m, n_experts, top_k), CS = shared ? (m + kChunk - 1) / kChunk : 0;
-  hipLaunchKernelGGL(prefill_group_kernel, dim3((unsigned)n_experts + 1), dim3(kThreads), 0, st, p);
+  p.n_sh_gu = shared ? (int)((m + kBigChunk - 1) / kBigChunk) : 0;
+  p.n_sh_dn = shared ? (int)((m + kChunk - 1) / kChunk) : 0;
+  const int64_t C = max_routed_chunks(m, n_experts, top_k);
+  hipLaunchKernelGGL(prefill_group_kernel, dim3((unsigned)n_experts + 1), dim3(kGroupThreads), 0, st, p);
   int rc = check_launch(name);
   if (rc) return rc;
-  const dim3 blk(kThreads), gu((unsigned)(C * (i / kGuRows))), dn((unsigned)(C * (d / kDnRows)));
-  if (scale_kind == HSMOE_SCALE_E8M0) hipLaunchKernelGGL((prefill_gate_up_kernel<kFp4E8M0, false>), gu, blk, 0, st, p);
-  else hipLaunchKernelGGL((prefill_gate_up_kernel<kFp4F32, false>), gu, blk, 0, st, p);
+  const dim3 blk(kThreads), gu((unsigned)((C + p.n_sh_gu) * (i / kGuRows))),
+      dn((unsigned)((C + p.n_sh_dn) * (d / kDnRows)));
+  if (scale_kind == HSMOE_SCALE_E8M0) hipLaunchKernelGGL(prefill_gate_up_kernel<kFp4E8M0>, gu, blk, 0, st, p);
+  else hipLaunchKernelGGL(prefill_gate_up_kernel<kFp4F32>, gu, blk, 0, st, p);
   if ((rc = check_launch(name))) return rc;
-  if (CS) {
-    hipLaunchKernelGGL((prefill_gate_up_kernel<kFp8Block, true>), dim3((unsigned)(CS * (i / kGuRows))), blk, 0, st, p);
-    if ((rc = check_launch(name))) return rc;
-  }
-  if (scale_kind == HSMOE_SCALE_E8M0) hipLaunchKernelGGL((prefill_down_kernel<kFp4E8M0, false>), dn, blk, 0, st, p);
-  else hipLaunchKernelGGL((prefill_down_kernel<kFp4F32, false>), dn, blk, 0, st, p);
+  if (scale_kind == HSMOE_SCALE_E8M0) hipLaunchKernelGGL(prefill_down_kernel<kFp4E8M0>, dn, blk, 0, st, p);
+  else hipLaunchKernelGGL(prefill_down_kernel<kFp4F32>, dn, blk, 0, st, p);
   if ((rc = check_launch(name))) return rc;
-  if (CS) {
-    hipLaunchKernelGGL((prefill_down_kernel<kFp8Block, true>), dim3((unsigned)(CS * (d / kDnRows))), blk, 0, st, p);
-    if ((rc = check_launch(name))) return rc;
-  }
   hipLaunchKernelGGL(prefill_combine_kernel, dim3((unsigned)m, (unsigned)(d / (4 * kThreads))), dim3(kThreads), 0,
                      st, p);
   return check_launch(name);
