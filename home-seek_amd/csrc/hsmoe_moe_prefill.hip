@@ -15,7 +15,8 @@
 // (every token through every selected expert), only the (token, expert) pairs
 // that routing selects are computed.
 //
-// Launches (no host synchronisation):
+// Launches (no host synchronisation; "wide" below for the form that calls with
+// many pairs per expert take instead of gate_up and down):
 //   group    workgroup e buckets the pairs (t, j) routed to expert e, in (t, j)
 //            order (stable, deterministic); one more workgroup places the
 //            shared expert's M pairs.  Each bucket is cut into gate/up chunks
@@ -31,6 +32,9 @@
 //   down     grid (chunk, 128-row block of D), same pipeline over W2 (32 rows
 //            per wave) with the activation tile (hi and lo planes); writes one
 //            fp32 partial row per pair (no atomics).
+//   wide     the same two passes for the shared expert's chunks and those of
+//            routed experts with more than 32 pairs, on 32-row tiles (beside
+//            gate_up and down, which then take the other experts).
 //   combine  out[t] = partials of t's pairs in slot order, then the shared one.
 // The grids are sized for the most chunks the routing can produce; workgroups
 // past the actual count (read from the workspace) exit at once.
@@ -57,8 +61,9 @@ constexpr int kMaxPairs = 12288;  // m * top_k per call (LDS of the group kernel
 constexpr int kMaxExperts = 1024;
 
 struct Header {
-  int n_gu;  // gate/up chunks: the shared expert's, then the routed experts' (big ones' first)
-  int n_dn;  // down chunks: the shared expert's, then the routed experts'
+  int n_gu;   // gate/up chunks: the shared expert's, then the routed experts' (big ones' first)
+  int n_dn;   // down chunks: the shared expert's, then the routed experts'
+  int n_big;  // gate/up chunks of the shared expert and the big routed experts
 };
 
 struct PrefillParams {
@@ -85,16 +90,22 @@ struct PrefillParams {
   int n_experts;
   int m, d, i, top_k;
   int n_sh_gu, n_sh_dn;  // chunks of the shared expert's m pairs in either list
+  int small, big_chunk;  // an expert of more than `small` pairs is cut into chunks of big_chunk
+  int by_rows;           // wide kernels: every chunk placed on the XCDs by row block
+  int wide;              // the first n_big gate/up chunks go to the wide kernels, in both passes
   float limit;
 };
 
 // ---------------------------------------------------------------- group
 // Pairs per gate/up chunk of an expert with cnt pairs: an expert with more
-// than kChunk pairs is cut into chunks of kBigChunk, so that its W1 and W3
+// than p.small (kChunk) pairs is cut into chunks of kBigChunk, so that its W1 and W3
 // are streamed half as often; big experts' chunks come first, so that the
 // longer workgroups start first.  The down pass keeps chunks of kChunk (its
-// token tile's size), in expert order: a second list.
-__device__ __forceinline__ int chunk_size(int cnt) { return cnt > kChunk ? kBigChunk : kChunk; }
+// token tile's size), in expert order: a second list (the wide kernels and what
+// runs beside them take the gate/up list in both passes).
+__device__ __forceinline__ int chunk_size(const PrefillParams& p, int cnt) {
+  return cnt > p.small ? p.big_chunk : kChunk;
+}
 
 // Sum over the block of v (every thread passes its own value).
 template <int kWaves>
@@ -153,18 +164,21 @@ __global__ void __launch_bounds__(kGroupThreads) prefill_group_kernel(PrefillPar
   }
   __syncthreads();
   if (me == E) {
-    int pairs = 0, chunks = 0, dchunks = 0;
+    int pairs = 0, chunks = 0, dchunks = 0, small = 0;
     for (int e = threadIdx.x; e < E; e += kGroupThreads) {
       pairs += s_cnt[e];
-      chunks += (s_cnt[e] + chunk_size(s_cnt[e]) - 1) / chunk_size(s_cnt[e]);
+      chunks += (s_cnt[e] + chunk_size(p, s_cnt[e]) - 1) / chunk_size(p, s_cnt[e]);
+      small += s_cnt[e] > 0 && s_cnt[e] <= p.small;
       dchunks += (s_cnt[e] + kChunk - 1) / kChunk;
     }
     pairs = block_sum<kWaves>(pairs, s_red);
     chunks = block_sum<kWaves>(chunks, s_red);
     dchunks = block_sum<kWaves>(dchunks, s_red);
+    small = block_sum<kWaves>(small, s_red);
     if (threadIdx.x == 0) {
       p.hdr->n_gu = p.n_sh_gu + chunks;
       p.hdr->n_dn = p.n_sh_dn + dchunks;
+      p.hdr->n_big = p.n_sh_gu + chunks - small;
     }
     for (int q = threadIdx.x; q < P; q += kGroupThreads)
       if (s_e[q] == kNone) p.pidx[(q / K) * (K + 1) + q % K] = -1;
@@ -190,19 +204,19 @@ __global__ void __launch_bounds__(kGroupThreads) prefill_group_kernel(PrefillPar
   const int cnt = s_cnt[me];
   if (cnt == 0) return;  // uniform across the workgroup
   // chunks: the big experts' (expert order), then one per small expert (expert order)
-  const bool big = cnt > kChunk;
+  const bool big = cnt > p.small;
   int off = 0, choff = 0, dnoff = 0;
   for (int e = threadIdx.x; e < E; e += kGroupThreads) {
     const int c = s_cnt[e];
     if (e < me) off += c;
     if (e < me) dnoff += (c + kChunk - 1) / kChunk;
-    if (c > kChunk && (!big || e < me)) choff += (c + kBigChunk - 1) / kBigChunk;  // every big expert's chunks first
+    if (c > p.small && (!big || e < me)) choff += (c + p.big_chunk - 1) / p.big_chunk;  // every big expert's chunks first
     else if (!big && e < me && c > 0) ++choff;
   }
   off = block_sum<kWaves>(off, s_red);
   choff = p.n_sh_gu + block_sum<kWaves>(choff, s_red);
   dnoff = p.n_sh_dn + block_sum<kWaves>(dnoff, s_red);
-  const int cs = chunk_size(cnt);
+  const int cs = chunk_size(p, cnt);
   // this wave's share of the list: its hits, then their places
   const int per = (P + 64 * kWaves - 1) / (64 * kWaves) * 64;
   const int q_lo = min(wave * per, P), q_hi = min(q_lo + per, P);
@@ -249,13 +263,17 @@ struct Chunk {
   const uint64_t* ent;
 };
 
-// Chunk q of the gate/up list or (kDown) the down list.
-template <bool kDown>
+// Chunk q of the gate/up list or (kDown) the down list; beside the wide
+// kernels chunk q of the gate/up list's small experts, which both passes take
+// (one chunk of at most kChunk pairs each); kWide: of its big part.
+template <bool kDown, bool kWide = false>
 __device__ __forceinline__ bool load_chunk(const PrefillParams& p, int q, Chunk& ch) {
-  if (q >= (kDown ? p.hdr->n_dn : p.hdr->n_gu)) return false;
-  ch.e = kDown ? p.dn_e[q] : p.chunk_e[q];
-  ch.p0 = kDown ? p.dn_p0[q] : p.chunk_p0[q];
-  ch.n = kDown ? p.dn_n[q] : p.chunk_n[q];
+  if (!kWide && p.wide) q += p.hdr->n_big;
+  const bool dn = kDown && !p.wide;
+  if (q >= (kWide ? p.hdr->n_big : dn ? p.hdr->n_dn : p.hdr->n_gu)) return false;
+  ch.e = dn ? p.dn_e[q] : p.chunk_e[q];
+  ch.p0 = dn ? p.dn_p0[q] : p.chunk_p0[q];
+  ch.n = dn ? p.dn_n[q] : p.chunk_n[q];
   ch.shared = ch.e == p.n_experts;
   ch.ent = ch.shared ? p.shared : p.table + (int64_t)ch.e * 6;
   return true;
@@ -608,6 +626,343 @@ prefill_down_kernel(PrefillParams p) {
   else down_chunk<F == kFp4E8M0 ? kFp4E8M0Split : F, 3>(p, ch, r0, as);  // routed E8M0: cached scales
 }
 
+// ---------------------------------------------------------------- wide
+// Gate/up (kDown false) and down for calls whose experts hold many pairs: a
+// workgroup takes a chunk of up to 64 pairs and 128 rows of W1 and W3 (32 per
+// wave and matrix), or 256 rows of W2 (two tiles of 32 per wave), on
+// v_mfma_f32_32x32x16_bf16.  With the 16-row tiles above every 16-byte LDS read
+// feeds two 16x16x32 products, which takes the LDS as long as the matrix cores,
+// and every row block of 64 reads the tokens again; here a read feeds two
+// products of twice the size and half as many row blocks read the tokens.  Two
+// waves per SIMD (256 registers) hold 64 accumulators, the unit of weights
+// being multiplied and the next one, and the next token tile on its way to the
+// other half of the LDS: one barrier per stage, a step's LDS reads and decode
+// under the products of the step before.
+// Measured at 12288 pairs of 256 experts and 2048 of the shared one, d = 4096,
+// i = 2048: gate/up 720 us, down 570 (0.86 and 1.09 PFLOP/s of issued products;
+// 455 and 375 with no loads in the loop), a layer of 4096 tokens 3290 -> 2820.
+//
+// Columns: a K-chunk is 256 columns; lane (c, h) of a wave owns columns
+// 128h .. +127 of it, as 4 groups of 32 (16 bytes of FP4 each), so that its 4
+// E8M0 scales are one aligned word.  A weight unit is 64 bytes of a lane's
+// columns per matrix: all 4 groups in FP4, 2 in FP8, 1 in bf16.  A stage is an
+// LDS tile: 64 tokens x 256 columns (gate/up), or the hi and lo planes of
+// 64 pairs x 128 columns (down: groups 2t and 2t + 1 of either half).  The LDS
+// rows are unpadded, 16-byte unit u of row t stored at u ^ (t & 15).
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kWideGuRows = 128;  // rows of W1 and W3 per workgroup
+constexpr int kWideDnRows = 256;  // rows of W2 per workgroup
+constexpr int kStage16 = 2048;    // 16-byte units per LDS stage
+
+__device__ __forceinline__ uint4 bload128s(BufRsrc r, uint32_t off, uint32_t soff) {
+  const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, (int)soff, 0);
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+
+// Dword v of q, v a constant after unrolling.
+__device__ __forceinline__ uint32_t dword(const uint4& q, int v) {
+  return v == 0 ? q.x : v == 1 ? q.y : v == 2 ? q.z : q.w;
+}
+
+// One exchange of a transpose over lanes: `odd` lanes give a and take the
+// other lane's b for it, the others give b and take a (kCtrl: the quad_perm
+// that names the other lane).
+template <int kCtrl>
+__device__ __forceinline__ void swap_pieces(uint4& a, uint4& b, bool odd) {
+  auto one = [odd](uint32_t& x, uint32_t& y) {
+    // (both moves run on every lane: they read the other's register)
+    const uint32_t ox = (uint32_t)__builtin_amdgcn_mov_dpp((int)x, kCtrl, 0xf, 0xf, true);
+    const uint32_t oy = (uint32_t)__builtin_amdgcn_mov_dpp((int)y, kCtrl, 0xf, 0xf, true);
+    x = odd ? oy : x;
+    y = odd ? y : ox;
+  };
+  one(a.x, b.x);
+  one(a.y, b.y);
+  one(a.z, b.z);
+  one(a.w, b.w);
+}
+
+// A unit of both matrices (or row tiles), its fp32 scales beside it.
+template <int F>
+struct WideUnit {
+  static constexpr int kUnits = F == kBf16 ? 4 : F == kFp8Block ? 2 : 1;  // per K-chunk
+  static constexpr int kGroups = 4 / kUnits;                              // of 32 columns, per half
+  static constexpr int kChunkBytes = 256 * kUnits / 2;                    // of a row, per K-chunk
+  uint4 q[2][4];
+  uint4 sf[2];  // kFp4F32: the 4 groups' scales
+  float s8[2];  // kFp8Block: the half's block scale
+  // q[t][v]: bytes 16 (c % 4) .. +15 of the unit of row 4 (c / 4) + v (wo: that
+  // of v = 0), so that four neighbouring lanes read one 64-byte run (a lane per
+  // row touches four times as many lines per load: a layer of 4096 tokens 2970
+  // us against 2856); turn() then gives lane c its own row's 64 bytes.
+  __device__ __forceinline__ void load(const Mat (&m)[2], const uint32_t (&wo)[2], const uint32_t (&so)[2], int kc,
+                                       int u, int row_bytes) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        q[t][v] = bload128s(m[t].w, wo[t] + 64 * u, (uint32_t)kc * kChunkBytes + (uint32_t)(v * row_bytes));
+      if constexpr (F == kFp4F32) sf[t] = bload128s(m[t].s, so[t], (uint32_t)kc * 32);
+      if constexpr (F == kFp8Block)
+        s8[t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(m[t].s, (int)so[t], kc * 8, 0));
+    }
+  }
+  // 4 x 4 transpose of the 16-byte pieces over each quad of lanes
+  __device__ __forceinline__ void turn() {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      swap_pieces<0xB1>(q[t][0], q[t][1], (lane & 1) != 0);
+      swap_pieces<0xB1>(q[t][2], q[t][3], (lane & 1) != 0);
+      swap_pieces<0x4E>(q[t][0], q[t][2], (lane & 2) != 0);
+      swap_pieces<0x4E>(q[t][1], q[t][3], (lane & 2) != 0);
+    }
+  }
+  // columns 8j .. +7 of the unit's group s (group gi of the half); e: the half's 4 E8M0 bytes
+  __device__ __forceinline__ bf16x8 frag(int t, int s, int gi, int j, uint32_t e) const {
+    if constexpr (F == kFp4E8M0) {
+      return fp4x8_to_bf16_e8m0(dword(q[t][s], j), e8m0_as_f32((e >> (8 * gi)) & 0xffu));
+    } else if constexpr (F == kFp4F32) {
+      return fp4x8_to_bf16_f32(dword(q[t][s], j), __uint_as_float(dword(sf[t], gi)));
+    } else if constexpr (F == kFp8Block) {
+      const uint4& w = q[t][2 * s + j / 2];
+      bf16x8 f;
+      fp8x4_to_bf16(dword(w, 2 * (j & 1)), s8[t], f, 0);
+      fp8x4_to_bf16(dword(w, 2 * (j & 1) + 1), s8[t], f, 1);
+      return f;
+    } else {
+      return __builtin_bit_cast(bf16x8, q[t][j]);
+    }
+  }
+};
+
+// The E8M0 bytes of 4 K-chunks: a lane reads 16 of a row's 32 bytes and the
+// two halves swap, so that w[q] is the lane's word of K-chunk q.
+struct WideScales {
+  uint32_t w[4];
+  __device__ __forceinline__ void deal(const uint4& raw) {
+    const auto a = __builtin_amdgcn_permlane32_swap(raw.x, raw.y, false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(raw.z, raw.w, false, false);
+    w[0] = a[0];
+    w[2] = a[1];
+    w[1] = b[0];
+    w[3] = b[1];
+  }
+};
+
+// One chunk's rows r0 .. of this wave; kTiles: 32-pair tiles of the chunk.
+template <int F, bool kDown, int kTiles>
+__device__ __forceinline__ void wide_chunk(const PrefillParams& p, const Chunk& ch, int r0, uint4* lds) {
+  using U = WideUnit<F>;
+  constexpr int kPlanes = kDown ? 2 : 1, kStages = kDown ? 2 : 1;  // planes per stage, stages per K-chunk
+  constexpr int kRow16 = kDown ? 16 : 32;                          // 16-byte units per LDS row
+  constexpr int kPer = kTiles * 32 * kRow16 / kThreads;            // units per thread and plane
+  constexpr int kStageGroups = 4 / kStages;
+  // units held: the one multiplied and those in flight (a bf16 unit is multiplied in 256 to 512 cycles, less
+  // than a load takes: three ahead where a chunk of one tile leaves the registers)
+  constexpr int kBufs = F == kBf16 && kTiles == 1 ? 4 : 2, kAhead = kBufs - 1;
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  const int K = kDown ? p.i : p.d, nkc = K / kCols, row_bytes = nkc * U::kChunkBytes;
+  // weights: W1 and W3 at one row, or W2 at two
+  Mat m[2];
+  uint32_t wo[2], so[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int slot = kDown ? 4 : 2 * t;
+    const uint32_t row = (uint32_t)(r0 + (kDown ? 32 * t : 0) + c);
+    m[t] = make_mat<F>(ch.ent[slot], ch.ent[slot + 1], kDown ? p.d : p.i, K);
+    wo[t] = (row - c % 4) * (uint32_t)row_bytes + h * (U::kChunkBytes / 2) + c % 4 * 16;
+    if constexpr (F == kFp4E8M0) so[t] = row * (uint32_t)(K / 32) + 16 * h;
+    else if constexpr (F == kFp4F32) so[t] = 4 * (row * (uint32_t)(K / 32) + 4 * h);
+    else so[t] = 4 * (row / 128 * (uint32_t)(K / 128) + h);
+  }
+  // the token tile: rows past the chunk's pairs repeat its last one (their results are dropped)
+  uint32_t xo[kPer];
+  uint4 xr[kPlanes][kPer];
+#pragma unroll
+  for (int v = 0; v < kPer; ++v) {
+    const int q = (int)threadIdx.x + v * kThreads, un = q % kRow16, src = min(q / kRow16, ch.n - 1);
+    if constexpr (kDown) xo[v] = 2 * ((uint32_t)src * (uint32_t)p.i + (un >> 3) * 128 + (un & 7) * 8);
+    else xo[v] = 2 * ((uint32_t)p.pair_tok[ch.p0 + src] * (uint32_t)p.d + un * 8);
+  }
+  BufRsrc xb[kPlanes];
+  if constexpr (kDown) {
+    xb[0] = make_buf((uint64_t)(p.act_hi + (int64_t)ch.p0 * p.i), 2u * ch.n * p.i);
+    xb[1] = make_buf((uint64_t)(p.act_lo + (int64_t)ch.p0 * p.i), 2u * ch.n * p.i);
+  } else {
+    xb[0] = make_buf((uint64_t)p.x, 2u * p.m * p.d);
+  }
+  // this thread's first unit of the LDS tile; its later ones are 8 (gate/up) or 16 rows on
+  const int x_row = (int)threadIdx.x / kRow16, x_un = (int)threadIdx.x % kRow16;
+  const int xl0 = x_row * kRow16 + (x_un ^ (x_row & 15)), xl1 = kDown ? xl0 : xl0 ^ 8;
+  auto xload = [&](int kc, int st) {
+#pragma unroll
+    for (int pl = 0; pl < kPlanes; ++pl)
+#pragma unroll
+      for (int v = 0; v < kPer; ++v) xr[pl][v] = bload128s(xb[pl], xo[v], (uint32_t)(kc * kCols + st * 64) * 2);
+  };
+  auto xstore = [&](int buf) {
+#pragma unroll
+    for (int pl = 0; pl < kPlanes; ++pl)
+#pragma unroll
+      for (int v = 0; v < kPer; ++v)
+        lds[buf * kStage16 + pl * (kStage16 / 2) + (v & 1 ? xl1 : xl0) + v * kThreads] = xr[pl][v];
+  };
+  f32x16 acc[2][kTiles];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int tile = 0; tile < kTiles; ++tile)
+#pragma unroll
+      for (int q = 0; q < 16; ++q) acc[t][tile][q] = 0.0f;
+  U w[kBufs];
+  uint4 raw[2];
+  WideScales sc[2];
+  xload(0, 0);
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) w[u].load(m, wo, so, 0, u, row_bytes);
+  if constexpr (F == kFp4E8M0) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) raw[t] = bload128(m[t].s, so[t]);
+  }
+  xstore(0);
+  // 16-byte unit of (group 0, j = 0) of this lane's columns in LDS row c; the
+  // others differ from it in the low bits only
+  const int lb = c * kRow16 + ((h * (kRow16 / 2)) ^ (c & 15));
+  for (int kc = 0; kc < nkc; kc += 2) {  // (K is a multiple of 512)
+    if constexpr (F == kFp4E8M0) {
+      if ((kc & 2) == 0) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) sc[t].deal(raw[t]);
+      } else {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          sc[t].w[0] = sc[t].w[2];
+          sc[t].w[1] = sc[t].w[3];
+          raw[t] = bload128(m[t].s, so[t] + (uint32_t)(kc + 2) * 8);  // (past the row or the end: unused)
+        }
+      }
+    }
+#pragma unroll
+    for (int k2 = 0; k2 < 2; ++k2) {
+#pragma unroll
+      for (int st = 0; st < kStages; ++st) {
+        const int buf = (k2 * kStages + st) & 1;
+        const bool last = k2 == 1 && st == kStages - 1;
+        const bool more = !last || kc + 2 < nkc;
+        __syncthreads();
+        if (more) xload(st == kStages - 1 ? kc + k2 + 1 : kc + k2, st == kStages - 1 ? 0 : st + 1);
+        const uint4* const tile16 = lds + buf * kStage16;
+        // steps of the stage: (group, j, plane); step k + 1's operands are read
+        // and decoded while step k is multiplied
+        constexpr int kSteps = kStageGroups * 4 * kPlanes;
+        bf16x8 a[2][2], bt[2][kTiles];
+        auto read_b = [&](int k) {
+          const int un = lb ^ (k / kPlanes), pl = k % kPlanes;
+#pragma unroll
+          for (int tile = 0; tile < kTiles; ++tile)
+            bt[k & 1][tile] =
+                *reinterpret_cast<const bf16x8*>(tile16 + pl * (kStage16 / 2) + tile * 32 * kRow16 + un);
+        };
+        auto decode = [&](int k) {  // k: (group, j)
+          const int gi = st * kStageGroups + k / 4, u = gi / U::kGroups;
+          U& wc = w[(k2 * U::kUnits + u) % kBufs];
+          if (gi % U::kGroups == 0 && k % 4 == 0) wc.turn();  // (the unit's first use)
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+            a[k & 1][t] = wc.frag(t, gi % U::kGroups, gi, k % 4, F == kFp4E8M0 ? sc[t].w[k2] : 0u);
+        };
+        read_b(0);
+        decode(0);
+#pragma unroll
+        for (int k = 0; k < kSteps; ++k) {
+          const int kd = k / kPlanes, gi = st * kStageGroups + kd / 4, u = gi / U::kGroups;
+          if (k % (4 * kPlanes) == 0 && gi % U::kGroups == 0) {  // a unit's first step: the weights of the unit kAhead on
+            const int un = k2 * U::kUnits + u + kAhead, ahead = un / U::kUnits;  // (counted from K-chunk kc)
+            if (ahead < 2 || kc + 2 < nkc) w[un % kBufs].load(m, wo, so, kc + ahead, un % U::kUnits, row_bytes);
+            __builtin_amdgcn_sched_barrier(0);  // (the scheduler would sink the loads to their uses)
+          }
+          if (k + 1 < kSteps) read_b(k + 1);
+          if (k % kPlanes == kPlanes - 1 && k + 1 < kSteps) decode(kd + 1);
+#pragma unroll
+          for (int tile = 0; tile < kTiles; ++tile)
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+              acc[t][tile] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kd & 1][t], bt[k & 1][tile], acc[t][tile], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (more) xstore(buf ^ 1);
+      }
+    }
+  }
+  // lane (c, h) holds rows 8 (q / 4) + 4h + q % 4 of pair 32 tile + c
+#pragma unroll
+  for (int tile = 0; tile < kTiles; ++tile) {
+    const int tt = tile * 32 + c;
+    if (tt >= ch.n) continue;
+    const int64_t pr = ch.p0 + tt;
+    if constexpr (kDown) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int q = 0; q < 16; q += 4)
+          *reinterpret_cast<float4*>(p.part + pr * p.d + r0 + 32 * t + 2 * q + 4 * h) =
+              make_float4(acc[t][tile][q], acc[t][tile][q + 1], acc[t][tile][q + 2], acc[t][tile][q + 3]);
+    } else {
+      const float wt = p.pair_w[pr];
+#pragma unroll
+      for (int q = 0; q < 16; q += 4) {
+        uint32_t hi[4], lo[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float a = __fmul_rn(wt, swiglu(acc[0][tile][q + v], acc[1][tile][q + v], p.limit));
+          hi[v] = f32_to_bf16_bits(a);
+          lo[v] = f32_to_bf16_bits(__fadd_rn(a, -bf16_bits_to_f32(hi[v])));
+        }
+        const int64_t o = pr * p.i + r0 + 2 * q + 4 * h;
+        *reinterpret_cast<uint2*>(p.act_hi + o) = make_uint2(hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16));
+        *reinterpret_cast<uint2*>(p.act_lo + o) = make_uint2(lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16));
+      }
+    }
+  }
+}
+
+template <int F, bool kDown>
+__device__ __forceinline__ void wide_any(const PrefillParams& p, const Chunk& ch, int r0, uint4* lds) {
+  if (ch.n > 32) wide_chunk<F, kDown, 2>(p, ch, r0, lds);
+  else wide_chunk<F, kDown, 1>(p, ch, r0, lds);
+}
+
+// F: format of the routed FP4 experts of the call's scale kind.
+template <int F, bool kDown>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+prefill_wide_kernel(PrefillParams p) {
+  __shared__ uint4 lds[2 * kStage16];
+  constexpr int kRows = kDown ? kWideDnRows : kWideGuRows;
+  // Workgroup b runs on XCD b % 8.  A routed chunk's row blocks go to one XCD,
+  // whose L2 then holds the chunk's tokens.  Chunks of one expert (the shared
+  // one's, or those of a call with few experts) go row block by row block, so
+  // that an XCD's L2 holds its share of the weights for all of them.
+  const int nrb = (kDown ? p.d : p.i) / kRows, n_rows = p.by_rows ? p.hdr->n_big * nrb : p.n_sh_gu * nrb;
+  int q, rb;
+  if ((int)blockIdx.x < n_rows) {
+    q = blockIdx.x / nrb;
+    rb = blockIdx.x % nrb;
+  } else {
+    const int b = blockIdx.x - n_rows, b8 = b / 8;
+    q = p.n_sh_gu + b8 / nrb * 8 + b % 8;
+    rb = b8 % nrb;
+  }
+  Chunk ch;
+  if (p.by_rows && (int)blockIdx.x >= n_rows) return;
+  if (!load_chunk<kDown, true>(p, q, ch)) return;
+  const int r0 = rb * kRows + kRows / 4 * (threadIdx.x >> 6);
+  if (!ch.ent[1]) wide_any<kBf16, kDown>(p, ch, r0, lds);
+  else if (ch.shared) wide_any<kFp8Block, kDown>(p, ch, r0, lds);
+  else wide_any<F, kDown>(p, ch, r0, lds);
+}
+
 // ---------------------------------------------------------------- combine
 // grid (m, d / 1024): thread -> 4 consecutive columns of one token.
 __global__ void __launch_bounds__(kThreads) prefill_combine_kernel(PrefillParams p) {
@@ -748,18 +1103,57 @@ extern "C" int hsmoe_moe_prefill(const void* x, int64_t m, int64_t d, int64_t i,
   hipStream_t st = (hipStream_t)stream;
   p.n_sh_gu = shared ? (int)((m + kBigChunk - 1) / kBigChunk) : 0;
   p.n_sh_dn = shared ? (int)((m + kChunk - 1) / kChunk) : 0;
-  const int64_t C = max_routed_chunks(m, n_experts, top_k);
+  const int64_t pk = m * top_k, touched = n_experts < pk ? n_experts : pk;
+  // The wide kernels take calls of 24 pairs per expert and more whose chunks
+  // fill the chip about four times (two workgroups per CU, i / 128 or d / 256
+  // of them per chunk of ~48 pairs), and every call of one expert with more
+  // than a chunk of pairs.  Small / wide kernels, us, d = 4096, i = 2048: 256
+  // experts of 12, 16, 23, 32 and 47 pairs 844 / 867, 925 / 927, 1060 / 1018,
+  // 1307 / 1195, 1640 / 1388; 64 experts of 28 pairs (two rounds of
+  // workgroups) 319 / 358; one bf16 expert of 40, 500 and 4096 pairs 154 / 117,
+  // 170 / 122, 836 / 407.  One expert's chunks are of 32 pairs where those give
+  // at most one workgroup per CU (500 pairs: 122, of 64 pairs 151; 1024 pairs of
+  // 64 158, 1023 of 32 192).
+  const bool one = n_experts == 1;
+  p.wide = one ? pk > kChunk : pk >= 24 * n_experts && pk * i >= (int64_t)12288 * 1024;
+  p.small = p.wide && one ? 0 : kChunk;
+  const int64_t blocks = i / kWideGuRows > d / kWideDnRows ? i / kWideGuRows : d / kWideDnRows;
+  p.big_chunk = p.wide && one && (pk + kChunk - 1) / kChunk * blocks <= 256 ? kChunk : kBigChunk;
+  p.by_rows = n_experts < 8;
+  // chunks of the small kernels (beside the wide ones at most one per expert), and of the wide ones
+  const int64_t C = p.wide ? (p.small ? touched : 0) : p.n_sh_gu + max_routed_chunks(m, n_experts, top_k);
+  const int64_t Cd = p.wide ? C : p.n_sh_dn + max_routed_chunks(m, n_experts, top_k);
+  const int64_t n_bigs = pk / (p.small + 1) < touched ? pk / (p.small + 1) : touched;
+  const int64_t big = p.wide ? p.n_sh_gu + (pk / p.big_chunk + n_bigs + 7) / 8 * 8 : 0;
   hipLaunchKernelGGL(prefill_group_kernel, dim3((unsigned)n_experts + 1), dim3(kGroupThreads), 0, st, p);
   int rc = check_launch(name);
   if (rc) return rc;
-  const dim3 blk(kThreads), gu((unsigned)((C + p.n_sh_gu) * (i / kGuRows))),
-      dn((unsigned)((C + p.n_sh_dn) * (d / kDnRows)));
-  if (scale_kind == HSMOE_SCALE_E8M0) hipLaunchKernelGGL(prefill_gate_up_kernel<kFp4E8M0>, gu, blk, 0, st, p);
-  else hipLaunchKernelGGL(prefill_gate_up_kernel<kFp4F32>, gu, blk, 0, st, p);
-  if ((rc = check_launch(name))) return rc;
-  if (scale_kind == HSMOE_SCALE_E8M0) hipLaunchKernelGGL(prefill_down_kernel<kFp4E8M0>, dn, blk, 0, st, p);
-  else hipLaunchKernelGGL(prefill_down_kernel<kFp4F32>, dn, blk, 0, st, p);
-  if ((rc = check_launch(name))) return rc;
+  const dim3 blk(kThreads);
+  const bool e8m0 = scale_kind == HSMOE_SCALE_E8M0;
+  if (big > 0) {
+    const dim3 gu((unsigned)(big * (i / kWideGuRows)));
+    if (e8m0) hipLaunchKernelGGL((prefill_wide_kernel<kFp4E8M0, false>), gu, blk, 0, st, p);
+    else hipLaunchKernelGGL((prefill_wide_kernel<kFp4F32, false>), gu, blk, 0, st, p);
+    if ((rc = check_launch(name))) return rc;
+  }
+  if (C > 0) {
+    const dim3 gu((unsigned)(C * (i / kGuRows)));
+    if (e8m0) hipLaunchKernelGGL(prefill_gate_up_kernel<kFp4E8M0>, gu, blk, 0, st, p);
+    else hipLaunchKernelGGL(prefill_gate_up_kernel<kFp4F32>, gu, blk, 0, st, p);
+    if ((rc = check_launch(name))) return rc;
+  }
+  if (big > 0) {
+    const dim3 dn((unsigned)(big * (d / kWideDnRows)));
+    if (e8m0) hipLaunchKernelGGL((prefill_wide_kernel<kFp4E8M0, true>), dn, blk, 0, st, p);
+    else hipLaunchKernelGGL((prefill_wide_kernel<kFp4F32, true>), dn, blk, 0, st, p);
+    if ((rc = check_launch(name))) return rc;
+  }
+  if (C > 0) {
+    const dim3 dn((unsigned)(Cd * (d / kDnRows)));
+    if (e8m0) hipLaunchKernelGGL(prefill_down_kernel<kFp4E8M0>, dn, blk, 0, st, p);
+    else hipLaunchKernelGGL(prefill_down_kernel<kFp4F32>, dn, blk, 0, st, p);
+    if ((rc = check_launch(name))) return rc;
+  }
   hipLaunchKernelGGL(prefill_combine_kernel, dim3((unsigned)m, (unsigned)(d / (4 * kThreads))), dim3(kThreads), 0,
                      st, p);
   return check_launch(name);

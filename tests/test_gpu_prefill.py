@@ -199,3 +199,44 @@ def test_full_shape_m512_zipf(dev):
         ops.moe_decode(x[a:a + 8], ti[a:a + 8], tw[a:a + 8], model.store.table(0), ops.SCALE_E8M0,
                        model.store.shared_entry(0), 10.0, out_f32=dec[a:a + 8], d=model.d, i=model.i)
     check_close(f32.cpu().numpy(), orc.to_np_bf16(out), dec.cpu().numpy(), "M=512 vs decode kernels")
+
+
+@pytest.fixture(scope="module")
+def odd(dev):
+    m = Model(dev, 9, 1024, 1536)  # 6 K-chunks in the down pass: its last read of scales is a half one
+    torch.cuda.synchronize()
+    return m
+
+
+@pytest.mark.parametrize("kind", ["e8m0", "f32", "bf16"])
+@pytest.mark.parametrize("n_exp,m,shared", [(1, 33, False), (1, 500, False), (1, 1089, True), (2, 40, True),
+                                            (9, 131, True)])
+def test_wide_kernels_every_format(odd, dev, kind, n_exp, m, shared):
+    """Calls whose experts hold many pairs (the 32-row kernels): every weight format, chunks of one and two
+    32-pair tiles with ragged ends, one expert (chunks of 32 below 1024 pairs, else 64), chunks placed by row
+    block (fewer than 8 experts) or by chunk, small experts beside big ones (ids 7 and 8 of 9)."""
+    k = 1 if n_exp < 3 else 2
+    entries = []
+    for e in range(n_exp):
+        w1, s1, w3, s3, w2, s2 = odd.store.expert_views(0, e)
+        if kind == "bf16":
+            entries.append(tuple(ops.fp4_dequant_bf16(a, b) for a, b in ((w1, s1), (w3, s3), (w2, s2))))
+        elif kind == "f32":
+            entries.append((w1, s1.to(torch.float32), w3, s3.to(torch.float32), w2, s2.to(torch.float32)))
+        else:
+            entries.append((w1, s1, w3, s3, w2, s2))
+    table = ops.expert_table(entries, dev)
+    x = synthetic.hidden(SEED, 40 + m, m, odd.d, dev)
+    idx = np.stack([(np.arange(m) * (j + 1) + j) % min(n_exp, 7) for j in range(k)], axis=1).astype(np.int64)
+    if n_exp == 9:
+        idx[:5, 0], idx[5:38, 1] = 7, 8  # a small expert and one of 33 pairs
+    if k == 2:
+        idx[idx[:, 0] == idx[:, 1], 1] = -1
+    w = np.linspace(0.2, 1.1, m * k, dtype=np.float32).reshape(m, k)
+    f32 = torch.empty(m, odd.d, dtype=torch.float32, device=dev)
+    out, _ = ops.moe_prefill(x, torch.as_tensor(idx, device=dev), torch.as_tensor(w, device=dev), table,
+                             ops.SCALE_F32 if kind == "f32" else ops.SCALE_E8M0,
+                             odd.store.shared_entry(0) if shared else None, 10.0, out_f32=f32, i=odd.i)
+    sample = np.unique(np.r_[0:m:7, 30:34, m - 3:m] % m)
+    ref = odd.oracle(x[sample], idx[sample], w[sample], shared=shared)
+    check_close(f32[sample].cpu().numpy(), orc.to_np_bf16(out[sample]), ref, f"wide {kind} E={n_exp} m={m}")
