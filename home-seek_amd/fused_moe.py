@@ -28,12 +28,35 @@ from . import ops
 from ._lib import SCALE_E8M0, SCALE_F32
 
 
+_FP4_DTYPES = (torch.int8, torch.uint8)
+_SCALE_KINDS = {torch.float8_e8m0fnu: SCALE_E8M0, torch.float32: SCALE_F32}
+
+
 def _as_device(t: torch.Tensor, dev: torch.device) -> torch.Tensor:
     return t if t.device == dev else t.to(dev, non_blocking=True)
 
 
+def _ready(w: tuple, dev: torch.device) -> bool:
+    """Every tensor of the entry is contiguous on a GPU `dev` (get_device instead of device: no object per tensor)."""
+    if dev.type != "cuda":
+        return False
+    index = dev.index
+    for t in w:
+        if t.get_device() != index or not t.is_contiguous():
+            return False
+    return True
+
+
 def _fp4_entry(w: tuple, dev: torch.device):
-    """Normalises a reference 6-tuple; returns (entry tuple, scale_kind)."""
+    """Normalises a reference 6-tuple; returns (entry tuple, scale_kind).
+
+    A tuple that needs nothing (contiguous on the device, E8M0 or fp32 scales)
+    is taken as it is: a call of FusedMoEFFN.forward makes one entry per
+    expert while the GPU waits for them all."""
+    if (w[0].dtype in _FP4_DTYPES and w[2].dtype in _FP4_DTYPES and w[4].dtype in _FP4_DTYPES
+            and w[1].dtype in _SCALE_KINDS and w[3].dtype == w[1].dtype and w[5].dtype == w[1].dtype
+            and _ready(w, dev)):
+        return tuple(w), _SCALE_KINDS[w[1].dtype]
     w1, s1, w3, s3, w2, s2 = (_as_device(t, dev) for t in w)
     kinds = set()
     out = []
@@ -106,7 +129,7 @@ class FusedMoEFFN:
         output is zeros when no expert remains.  Exceptions propagate."""
         B, D = hidden_states.shape
         dev = hidden_states.device
-        ids = sorted({int(e) for e in topk_idx.reshape(-1).tolist() if int(e) >= 0})
+        ids = sorted({int(e) for e in set(topk_idx.reshape(-1).tolist()) if int(e) >= 0})
         if not ids:
             return torch.zeros_like(hidden_states)
         entries: list = [None] * (max(ids) + 1)

@@ -7,6 +7,7 @@ zero, so stream-ordered calls can share them.
 """
 from __future__ import annotations
 
+import array
 import ctypes
 
 import torch
@@ -165,19 +166,25 @@ def expert_table(entries: list, device: torch.device) -> torch.Tensor:
 
     An entry is None (absent expert), a 6-tuple (w1, s1, w3, s3, w2, s2) of FP4
     tensors, or a 3-tuple (w1, w3, w2) of bf16 tensors."""
-    rows = []
+    flat = array.array("q")
     for ent in entries:
         if ent is None:
-            rows.append([0] * 6)
+            flat.extend((0, 0, 0, 0, 0, 0))
         elif len(ent) == 6:
-            rows.append([t.data_ptr() for t in ent])
+            flat.extend([t.data_ptr() for t in ent])
         elif len(ent) == 3:
             w1, w3, w2 = ent
-            rows.append([w1.data_ptr(), 0, w3.data_ptr(), 0, w2.data_ptr(), 0])
+            flat.extend((w1.data_ptr(), 0, w3.data_ptr(), 0, w2.data_ptr(), 0))
         else:
             raise ValueError(f"expert entry of length {len(ent)}")
-    host = torch.tensor(rows, dtype=torch.int64)
-    return host.to(device, non_blocking=False)
+    if not flat:
+        return torch.empty(0, dtype=torch.int64, device=device)
+    rows = torch.frombuffer(flat, dtype=torch.int64).reshape(-1, 6)
+    # through pinned memory (torch's cached host allocator keeps it until the
+    # copy is done): the copy of a pageable tensor waits for the whole stream
+    if torch.device(device).type == "cuda":
+        rows = rows.pin_memory()
+    return rows.to(device, non_blocking=True)
 
 
 def shared_entry(w1, s1, w3, s3, w2, s2, device: torch.device) -> torch.Tensor:
