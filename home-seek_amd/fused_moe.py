@@ -53,7 +53,7 @@ def _fp4_entry(w: tuple, dev: torch.device):
     A tuple that needs nothing (contiguous on the device, E8M0 or fp32 scales)
     is taken as it is: a call of FusedMoEFFN.forward makes one entry per
     expert while the GPU waits for them all."""
-    if (w[0].dtype in _FP4_DTYPES and w[2].dtype in _FP4_DTYPES and w[4].dtype in _FP4_DTYPES
+    if (len(w) == 6 and w[0].dtype in _FP4_DTYPES and w[2].dtype in _FP4_DTYPES and w[4].dtype in _FP4_DTYPES
             and w[1].dtype in _SCALE_KINDS and w[3].dtype == w[1].dtype and w[5].dtype == w[1].dtype
             and _ready(w, dev)):
         return tuple(w), _SCALE_KINDS[w[1].dtype]

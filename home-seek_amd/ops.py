@@ -181,8 +181,12 @@ def expert_table(entries: list, device: torch.device) -> torch.Tensor:
         return torch.empty(0, dtype=torch.int64, device=device)
     rows = torch.frombuffer(flat, dtype=torch.int64).reshape(-1, 6)
     # through pinned memory (torch's cached host allocator keeps it until the
-    # copy is done): the copy of a pageable tensor waits for the whole stream
+    # copy is done): the copy of a pageable tensor waits for the whole stream.
+    # A graph would read the pinned block again when others own it: refused
+    # under capture (as the waiting copy was).
     if torch.device(device).type == "cuda":
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("an expert table is made from host memory: not under graph capture")
         rows = rows.pin_memory()
     return rows.to(device, non_blocking=True)
 

@@ -144,6 +144,40 @@ def test_fused_moe_forward_with_reference_loaders(layer, dev):
     assert_bf16_close(orc.bf16_to_f32(orc.to_np_bf16(out)), orc.bf16_to_f32(orc.f32_to_bf16(ref)))
 
 
+@pytest.mark.parametrize("form", ["strided", "host", "bf16 scales"])
+def test_loader_entries_that_need_work(layer, dev, form):
+    """Entries that are not contiguous on the device in a taken scale type give the results of those that are."""
+    store, gate, bias = layer
+    moe = fused_moe.FusedMoEFFN(E, I, D, 10.0)
+    x = synthetic.hidden(SEED, 410, 2, D, dev)
+    idx, w = ops.router_topk(x, gate, bias, K, 1.5)
+
+    def ready(layer_idx, eid):
+        v = store.expert_views(0, eid)
+        return tuple(t if q % 2 == 0 else t.to(torch.float32) for q, t in enumerate(v))
+
+    def other(layer_idx, eid):
+        v = ready(layer_idx, eid)
+        if form == "strided":
+            return tuple(torch.stack((t.view(torch.uint8), t.view(torch.uint8)), dim=-1)[..., 0].view(torch.uint8)
+                         if q % 2 == 0 else torch.stack((t, t), dim=-1)[..., 0] for q, t in enumerate(v))
+        if form == "host":
+            return tuple(t.cpu() for t in v)
+        return tuple(t if q % 2 == 0 else t.to(torch.bfloat16) for q, t in enumerate(v))  # (powers of two: exact)
+
+    assert torch.equal(moe.forward(x, idx, w, other, 0), moe.forward(x, idx, w, ready, 0))
+
+
+def test_expert_table_stays_refused_under_capture(layer, dev, monkeypatch):
+    """The table is made from host memory: a graph that copied it would read it again on every replay."""
+    entries = [layer[0].expert_views(0, 0)]
+    with monkeypatch.context() as mp:
+        mp.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+        with pytest.raises(RuntimeError, match="capture"):
+            ops.expert_table(entries, dev)
+    assert int(ops.expert_table(entries, dev)[0, 0]) == entries[0][0].data_ptr()
+
+
 def test_forward_m1_fp4_dict_api(layer, dev):
     store, _, _ = layer
     moe = fused_moe.FusedMoEFFN(E, I, D, 10.0)
