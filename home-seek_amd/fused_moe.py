@@ -154,7 +154,7 @@ class FusedMoEFFN:
         if len(kinds) > 1:
             raise TypeError("experts of one call mix E8M0 and fp32 scales")
         kind = kinds.pop() if kinds else SCALE_E8M0
-        table = ops.expert_table(entries, dev)
+        table = ops.expert_table(entries, dev, wait=False)  # (read on this stream only)
         x = hidden_states.to(torch.bfloat16)
         out = _run_decode_chunks(x, topk_idx, topk_weights, table, kind, None, self.swiglu_limit, D, inter)
         return out.to(hidden_states.dtype)
@@ -175,7 +175,7 @@ class FusedMoEFFN:
             kinds.add(kind)
         if len(kinds) > 1:
             raise TypeError("experts of one call mix E8M0 and fp32 scales")
-        table = ops.expert_table(entries, dev)
+        table = ops.expert_table(entries, dev, wait=False)  # (read on this stream only)
         idx = torch.arange(len(eids), dtype=torch.int64).reshape(1, -1).to(dev)
         w = torch.tensor([[float(routing_w[e]) for e in eids]], dtype=torch.float32).to(dev)
         out, _ = ops.moe_decode(hidden_states.to(torch.bfloat16), idx, w, table, kinds.pop(), None,
@@ -226,7 +226,7 @@ def fused_expert_ffn_pt(hidden: torch.Tensor, w1: torch.Tensor, w3: torch.Tensor
     """One bf16 expert (fused_moe.py:383-395) as a weight-1 slot of the HIP FFN."""
     dev = hidden.device
     w1, w3, w2 = _bf16_entry((w1, w3, w2), dev)
-    table = ops.expert_table([(w1, w3, w2)], dev)
+    table = ops.expert_table([(w1, w3, w2)], dev, wait=False)
     m = hidden.shape[0]
     idx = torch.zeros(m, 1, dtype=torch.int64, device=dev)
     w = torch.ones(m, 1, dtype=torch.float32, device=dev)
@@ -248,7 +248,7 @@ def fused_expert_ffn_triton(hidden: torch.Tensor, w1: torch.Tensor, w3: torch.Te
     else:
         ent, kind = _bf16_entry((w1, w3, w2), dev), SCALE_E8M0
         inter = ent[0].shape[0]
-    table = ops.expert_table([ent], dev)
+    table = ops.expert_table([ent], dev, wait=False)
     m = hidden.shape[0]
     idx = torch.zeros(m, 1, dtype=torch.int64, device=dev)
     w = torch.ones(m, 1, dtype=torch.float32, device=dev)

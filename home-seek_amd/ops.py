@@ -161,11 +161,13 @@ def router_topk(x: torch.Tensor, gate_w: torch.Tensor, bias: torch.Tensor | None
     return (idx, w, logits) if want_logits else (idx, w)
 
 
-def expert_table(entries: list, device: torch.device) -> torch.Tensor:
+def expert_table(entries: list, device: torch.device, wait: bool = True) -> torch.Tensor:
     """uint64 [n][6] device table from per-expert tuples.
 
     An entry is None (absent expert), a 6-tuple (w1, s1, w3, s3, w2, s2) of FP4
-    tensors, or a 3-tuple (w1, w3, w2) of bf16 tensors."""
+    tensors, or a 3-tuple (w1, w3, w2) of bf16 tensors.
+    The table is on the device when this returns, for kernels on any stream;
+    with wait=False it is there for what the current stream runs next only."""
     flat = array.array("q")
     for ent in entries:
         if ent is None:
@@ -180,15 +182,16 @@ def expert_table(entries: list, device: torch.device) -> torch.Tensor:
     if not flat:
         return torch.empty(0, dtype=torch.int64, device=device)
     rows = torch.frombuffer(flat, dtype=torch.int64).reshape(-1, 6)
-    # through pinned memory (torch's cached host allocator keeps it until the
-    # copy is done): the copy of a pageable tensor waits for the whole stream.
-    # A graph would read the pinned block again when others own it: refused
-    # under capture (as the waiting copy was).
+    # The copy of a pageable tensor waits for the whole stream.  Without that
+    # wait: through pinned memory (torch's cached host allocator keeps it until
+    # the copy is done).  A graph would read the host memory again when others
+    # own it: refused under capture.
     if torch.device(device).type == "cuda":
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("an expert table is made from host memory: not under graph capture")
-        rows = rows.pin_memory()
-    return rows.to(device, non_blocking=True)
+        if not wait:
+            return rows.pin_memory().to(device, non_blocking=True)
+    return rows.to(device)
 
 
 def shared_entry(w1, s1, w3, s3, w2, s2, device: torch.device) -> torch.Tensor:

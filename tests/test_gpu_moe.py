@@ -178,6 +178,22 @@ def test_expert_table_stays_refused_under_capture(layer, dev, monkeypatch):
     assert int(ops.expert_table(entries, dev)[0, 0]) == entries[0][0].data_ptr()
 
 
+def test_expert_table_read_on_another_stream(layer, dev):
+    """The stream that is current when the table is made is busy; another one reads the table at once."""
+    entries = [layer[0].expert_views(0, e) for e in range(E)]
+    want = [[t.data_ptr() for t in ent] for ent in entries]
+    a = torch.randn(4096, 4096, device=dev)
+    torch.cuda.synchronize()
+    for _ in range(20):
+        a = a @ a
+    table = ops.expert_table(entries, dev)
+    side = torch.cuda.Stream(dev)
+    with torch.cuda.stream(side):
+        got = table.clone()
+    side.synchronize()
+    assert got.tolist() == want
+
+
 def test_forward_m1_fp4_dict_api(layer, dev):
     store, _, _ = layer
     moe = fused_moe.FusedMoEFFN(E, I, D, 10.0)
