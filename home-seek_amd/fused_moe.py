@@ -47,8 +47,15 @@ def _ready(w: tuple, dev: torch.device) -> bool:
     return True
 
 
+def _copied(w: tuple, dev: torch.device) -> bool:
+    """Some tensor of the entry comes from elsewhere (pinned host memory: its
+    copy may still be running when _as_device returns, and the caller may
+    refill the buffer once the call that uses it has returned)."""
+    return any(t.device != dev for t in w)
+
+
 def _fp4_entry(w: tuple, dev: torch.device):
-    """Normalises a reference 6-tuple; returns (entry tuple, scale_kind).
+    """Normalises a reference 6-tuple; returns (entry tuple, scale_kind, _copied).
 
     A tuple that needs nothing (contiguous on the device, E8M0 or fp32 scales)
     is taken as it is: a call of FusedMoEFFN.forward makes one entry per
@@ -56,7 +63,8 @@ def _fp4_entry(w: tuple, dev: torch.device):
     if (len(w) == 6 and w[0].dtype in _FP4_DTYPES and w[2].dtype in _FP4_DTYPES and w[4].dtype in _FP4_DTYPES
             and w[1].dtype in _SCALE_KINDS and w[3].dtype == w[1].dtype and w[5].dtype == w[1].dtype
             and _ready(w, dev)):
-        return tuple(w), _SCALE_KINDS[w[1].dtype]
+        return tuple(w), _SCALE_KINDS[w[1].dtype], False
+    copied = _copied(w, dev)
     w1, s1, w3, s3, w2, s2 = (_as_device(t, dev) for t in w)
     kinds = set()
     out = []
@@ -68,11 +76,12 @@ def _fp4_entry(w: tuple, dev: torch.device):
         out += [data.contiguous(), sc2.contiguous()]
     if len(kinds) != 1:
         raise TypeError("all three scales of one expert must share one dtype")
-    return tuple(out), kinds.pop()
+    return tuple(out), kinds.pop(), copied
 
 
 def _bf16_entry(w: tuple, dev: torch.device):
-    return tuple(_as_device(t, dev).to(torch.bfloat16).contiguous() for t in w)
+    """A reference 3-tuple as bf16 on the device; returns (entry tuple, _copied)."""
+    return tuple(_as_device(t, dev).to(torch.bfloat16).contiguous() for t in w), _copied(w, dev)
 
 
 def _run_decode_chunks(x: torch.Tensor, topk_idx: torch.Tensor, topk_w: torch.Tensor, table: torch.Tensor,
@@ -135,26 +144,29 @@ class FusedMoEFFN:
         entries: list = [None] * (max(ids) + 1)
         kinds = set()
         inter = None
+        wait = False
         for eid in ids:
             w = load_expert_fn(layer_idx, eid)
             if w is None:
                 continue
             if len(w) == 6:
-                ent, kind = _fp4_entry(w, dev)
+                ent, kind, copied = _fp4_entry(w, dev)
                 kinds.add(kind)
                 inter = ent[0].shape[0]
             elif len(w) == 3:
-                ent = _bf16_entry(w, dev)
+                ent, copied = _bf16_entry(w, dev)
                 inter = ent[0].shape[0]
             else:
                 continue
+            wait = wait or copied
             entries[eid] = ent
         if inter is None:
             return torch.zeros_like(hidden_states)
         if len(kinds) > 1:
             raise TypeError("experts of one call mix E8M0 and fp32 scales")
         kind = kinds.pop() if kinds else SCALE_E8M0
-        table = ops.expert_table(entries, dev, wait=False)  # (read on this stream only)
+        # read on this stream only; its wait is that for the entries' copies
+        table = ops.expert_table(entries, dev, wait=wait)
         x = hidden_states.to(torch.bfloat16)
         out = _run_decode_chunks(x, topk_idx, topk_weights, table, kind, None, self.swiglu_limit, D, inter)
         return out.to(hidden_states.dtype)
@@ -169,13 +181,15 @@ class FusedMoEFFN:
             return torch.zeros(1, D, dtype=torch.bfloat16, device=dev)
         entries = []
         kinds = set()
+        wait = False
         for e in eids:
-            ent, kind = _fp4_entry(fp4_data[e], dev)
+            ent, kind, copied = _fp4_entry(fp4_data[e], dev)
             entries.append(ent)
             kinds.add(kind)
+            wait = wait or copied
         if len(kinds) > 1:
             raise TypeError("experts of one call mix E8M0 and fp32 scales")
-        table = ops.expert_table(entries, dev, wait=False)  # (read on this stream only)
+        table = ops.expert_table(entries, dev, wait=wait)
         idx = torch.arange(len(eids), dtype=torch.int64).reshape(1, -1).to(dev)
         w = torch.tensor([[float(routing_w[e]) for e in eids]], dtype=torch.float32).to(dev)
         out, _ = ops.moe_decode(hidden_states.to(torch.bfloat16), idx, w, table, kinds.pop(), None,
@@ -225,8 +239,8 @@ def fused_expert_ffn_pt(hidden: torch.Tensor, w1: torch.Tensor, w3: torch.Tensor
                         swiglu_limit: float = 10.0) -> torch.Tensor:
     """One bf16 expert (fused_moe.py:383-395) as a weight-1 slot of the HIP FFN."""
     dev = hidden.device
-    w1, w3, w2 = _bf16_entry((w1, w3, w2), dev)
-    table = ops.expert_table([(w1, w3, w2)], dev, wait=False)
+    (w1, w3, w2), copied = _bf16_entry((w1, w3, w2), dev)
+    table = ops.expert_table([(w1, w3, w2)], dev, wait=copied)
     m = hidden.shape[0]
     idx = torch.zeros(m, 1, dtype=torch.int64, device=dev)
     w = torch.ones(m, 1, dtype=torch.float32, device=dev)
@@ -243,12 +257,12 @@ def fused_expert_ffn_triton(hidden: torch.Tensor, w1: torch.Tensor, w3: torch.Te
     if w1.dtype in (torch.int8, torch.uint8):
         if w1_scale is None or w3_scale is None or w2_scale is None:
             raise ValueError("FP4 weights need all three scales")
-        ent, kind = _fp4_entry((w1, w1_scale, w3, w3_scale, w2, w2_scale), dev)
+        ent, kind, copied = _fp4_entry((w1, w1_scale, w3, w3_scale, w2, w2_scale), dev)
         inter = ent[0].shape[0]
     else:
-        ent, kind = _bf16_entry((w1, w3, w2), dev), SCALE_E8M0
+        (ent, copied), kind = _bf16_entry((w1, w3, w2), dev), SCALE_E8M0
         inter = ent[0].shape[0]
-    table = ops.expert_table([ent], dev, wait=False)
+    table = ops.expert_table([ent], dev, wait=copied)
     m = hidden.shape[0]
     idx = torch.zeros(m, 1, dtype=torch.int64, device=dev)
     w = torch.ones(m, 1, dtype=torch.float32, device=dev)

@@ -168,6 +168,41 @@ def test_loader_entries_that_need_work(layer, dev, form):
     assert torch.equal(moe.forward(x, idx, w, other, 0), moe.forward(x, idx, w, ready, 0))
 
 
+@pytest.mark.parametrize("form", ["fp4 loader", "bf16 loader", "shared"])
+def test_pinned_weights_refilled_after_the_call(layer, dev, form):
+    """The call returns when it has read the host's weights, also behind a busy stream."""
+    store = layer[0]
+    fp4 = store.expert_views(0, 3)
+    src = fp4 if form == "fp4 loader" else tuple(ops.fp4_dequant_bf16(fp4[q], fp4[q + 1]) for q in (0, 2, 4))
+    x = synthetic.hidden(SEED, 411, 1, D, dev)
+    idx, w = torch.full((1, 1), 3, device=dev), torch.ones(1, 1, device=dev)
+    pinned = tuple(torch.empty(t.shape, dtype=t.dtype, pin_memory=True) for t in src)
+    busy = torch.randn(4096, 4096, device=dev)
+
+    def call(entry, before):
+        def load(layer_idx, eid):
+            before()
+            return entry
+        if form == "shared":
+            before()
+            return fused_moe.SharedExpertFFN(D, I, 10.0).forward(x[None], *entry)[0]
+        return fused_moe.FusedMoEFFN(E, I, D, 10.0).forward(x, idx, w, load, 0)
+
+    def work():
+        y = busy
+        for _ in range(20):
+            y = y @ busy
+
+    want = call(src, lambda: None)
+    for t, p in zip(src, pinned):
+        p.copy_(t)
+    torch.cuda.synchronize()
+    got = call(pinned, work)
+    for p in pinned:
+        p.view(torch.uint8).zero_()
+    assert torch.equal(got, want)
+
+
 def test_expert_table_stays_refused_under_capture(layer, dev, monkeypatch):
     """The table is made from host memory: a graph that copied it would read it again on every replay."""
     entries = [layer[0].expert_views(0, 0)]

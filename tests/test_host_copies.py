@@ -3,7 +3,7 @@ pin_memory are recorded in place of a GPU's."""
 import pytest
 import torch
 
-from home_seek_amd import ops
+from home_seek_amd import fused_moe, ops
 
 CUDA = torch.device("cuda", 0)
 
@@ -36,3 +36,33 @@ def test_expert_table_is_on_the_device_when_it_returns(copies):
     table = ops.expert_table([None, ent], CUDA)
     assert table.tolist() == [[0] * 6, [t.data_ptr() for t in ent]]
     assert copies == [(12, True)]
+
+
+def host_calls():
+    """The calls that take weights from the host, each on hidden states of another device."""
+    x = torch.zeros(1, 4, dtype=torch.bfloat16, device="meta")
+    fp4 = tuple(torch.zeros(4, 4, dtype=torch.int8) if q % 2 == 0 else torch.zeros(4, 4) for q in range(6))
+    bf16 = tuple(torch.zeros(4, 4, dtype=torch.bfloat16) for _ in range(3))
+    moe, idx, w = fused_moe.FusedMoEFFN(4, 4, 4), torch.zeros(1, 1, dtype=torch.int64), torch.ones(1, 1)
+    return {
+        "forward fp4": lambda to: moe.forward(x, idx, w, lambda layer, e: to(fp4), 0),
+        "forward bf16": lambda to: moe.forward(x, idx, w, lambda layer, e: to(bf16), 0),
+        "shared": lambda to: fused_moe.SharedExpertFFN(4, 4).forward(x[None], *to(bf16)),
+        "pt": lambda to: fused_moe.fused_expert_ffn_pt(x, *to(bf16)),
+        "triton bf16": lambda to: fused_moe.fused_expert_ffn_triton(x, *to(bf16)),
+        "triton fp4": lambda to: (lambda e: fused_moe.fused_expert_ffn_triton(
+            x, e[0], e[2], e[4], w1_scale=e[1], w3_scale=e[3], w2_scale=e[5]))(to(fp4)),
+    }
+
+
+@pytest.mark.parametrize("call", list(host_calls()))
+def test_host_weights_are_read_when_the_call_returns(call, monkeypatch):
+    """A caller may refill a pinned buffer after the call that took it; entries on the device are not waited for."""
+    waits = []
+    monkeypatch.setattr(ops, "expert_table", lambda entries, device, wait=True: waits.append(wait))
+    monkeypatch.setattr(fused_moe, "_run_decode_chunks", lambda x, *args, **kw: torch.empty_like(x))
+    run = host_calls()[call]
+    run(lambda entry: entry)
+    run(lambda entry: tuple(t.to("meta") for t in entry))
+    run(lambda entry: (entry[0].to("meta"), *entry[1:]))
+    assert waits == [True, False, True]
