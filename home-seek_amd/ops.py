@@ -187,7 +187,9 @@ def expert_table(entries: list, device: torch.device, wait: bool = True) -> torc
     # the copy is done).  A graph would read the host memory again when others
     # own it: refused under capture.
     if torch.device(device).type == "cuda":
-        if torch.cuda.is_current_stream_capturing():
+        with torch.cuda.device(device):  # the copy runs on this device's stream
+            capturing = torch.cuda.is_current_stream_capturing()
+        if capturing:
             raise RuntimeError("an expert table is made from host memory: not under graph capture")
         if not wait:
             return rows.pin_memory().to(device, non_blocking=True)

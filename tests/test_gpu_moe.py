@@ -213,6 +213,24 @@ def test_expert_table_stays_refused_under_capture(layer, dev, monkeypatch):
     assert int(ops.expert_table(entries, dev)[0, 0]) == entries[0][0].data_ptr()
 
 
+def test_expert_table_refused_in_a_real_capture(layer, dev):
+    """Refused before anything is recorded: the capture goes on and its graph replays."""
+    entries = [layer[0].expert_views(0, 0)]
+    x, y = torch.ones(4, device=dev), torch.zeros(4, device=dev)
+    torch.add(x, 1.0, out=y)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for wait in (True, False):
+            with pytest.raises(RuntimeError, match="capture"):
+                ops.expert_table(entries, dev, wait=wait)
+        torch.add(x, 1.0, out=y)
+    for rep in range(3):
+        x.fill_(float(rep))
+        graph.replay()
+        assert y.tolist() == [rep + 1.0] * 4
+
+
 def test_expert_table_read_on_another_stream(layer, dev):
     """The stream that is current when the table is made is busy; another one reads the table at once."""
     entries = [layer[0].expert_views(0, e) for e in range(E)]

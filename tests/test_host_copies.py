@@ -1,5 +1,7 @@
 """Which host-to-device copies the calls wait for, on the CPU: Tensor.to and
 pin_memory are recorded in place of a GPU's."""
+import contextlib
+
 import pytest
 import torch
 
@@ -9,7 +11,22 @@ CUDA = torch.device("cuda", 0)
 
 
 @pytest.fixture
-def copies(monkeypatch):
+def current(monkeypatch):
+    """The current device, as torch.cuda.device sets it."""
+    now = [0]
+
+    @contextlib.contextmanager
+    def device(d):
+        before, now[0] = now[0], torch.device(d).index
+        yield
+        now[0] = before
+
+    monkeypatch.setattr(torch.cuda, "device", device)
+    return now
+
+
+@pytest.fixture
+def copies(monkeypatch, current):
     """[(numel, waits)] of the copies to CUDA, in order; the tensors stay where they are."""
     log = []
     real = torch.Tensor.to
@@ -36,6 +53,17 @@ def test_expert_table_is_on_the_device_when_it_returns(copies):
     table = ops.expert_table([None, ent], CUDA)
     assert table.tolist() == [[0] * 6, [t.data_ptr() for t in ent]]
     assert copies == [(12, True)]
+
+
+def test_capture_is_asked_of_the_device_that_gets_the_table(copies, current, monkeypatch):
+    """The stream that copies is the table's device's, whichever device is current."""
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: current[0] == 1)
+    assert ops.expert_table([entry()], torch.device("cuda", 0)).shape == (1, 6)
+    with pytest.raises(RuntimeError, match="capture"):
+        ops.expert_table([entry()], torch.device("cuda", 1))
+    current[0] = 1  # a capture on the current device is no matter of the other one's
+    assert ops.expert_table([entry()], torch.device("cuda", 0)).shape == (1, 6)
+    assert len(copies) == 2
 
 
 def host_calls():
