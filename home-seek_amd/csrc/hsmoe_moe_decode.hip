@@ -162,7 +162,6 @@ __global__ void __launch_bounds__(64 * kP2Waves) moe_down_kernel(DecodeParams p)
   __shared__ int s_cand[kMaxCand];
   __shared__ int s_first[kMaxCand];
   __shared__ int s_last;
-  __shared__ bool s_sel[kMaxTok][kMaxCand + 1];
   build_plan(p, plan, s_cand, s_first);
   const int n_slots = plan.n_routed + (p.shared ? 1 : 0);
   const int s = blockIdx.y;
@@ -227,20 +226,27 @@ __global__ void __launch_bounds__(64 * kP2Waves) moe_down_kernel(DecodeParams p)
              (unsigned)(n_slots - 1);
   __syncthreads();
   if (!s_last) return;
-  // the slots a token selects (the shared one: every token); the other slots'
-  // partials of it are products with zero activations and stay out of its sum
-  for (int q = threadIdx.x; q < n_slots * p.m; q += blockDim.x) {
-    const int sl = q / p.m, t = q - sl * p.m;
-    bool sel = sl == plan.n_routed;
-    for (int k = 0; k < p.top_k && !sel; ++k) sel = p.idx[t * p.top_k + k] == plan.eid[sl];
-    s_sel[t][sl] = sel;
-  }
-  __syncthreads();
-  const int rows = 16 * kP2Waves;
-  for (int q = threadIdx.x; q < rows * p.m; q += blockDim.x) {
-    const int t = q / rows, d = blockIdx.x * rows + (q - t * rows);
-    const float v = sum_slots_agent(p.part + (int64_t)t * p.d + d, (int64_t)p.m * p.d, n_slots, s_sel[t]);
-    const int64_t o = (int64_t)t * p.d + d;
+  // Wave w adds the 64 rows of tokens w, w + kP2Waves, ... over the routed
+  // slots the token selects (the other slots' partials of it are products with
+  // zero activations and stay out of its sum), then the shared one.  The token's
+  // slots come from the plan's LDS as two ballots: looked up in topk_idx, or
+  // kept per (token, slot) in LDS, they cost 1 to 13 us a call.
+  static_assert(16 * kP2Waves == 64 && kMaxCand <= 128, "a lane per row; two words of slots");
+  const int64_t stride = (int64_t)p.m * p.d;
+  for (int t = wave; t < p.m; t += kP2Waves) {
+    const int64_t o = (int64_t)t * p.d + blockIdx.x * 64 + lane;
+    const float sv = p.shared ? load_agent(p.part + plan.n_routed * stride + o) : 0.0f;
+    uint64_t sel[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int sl = lane + 64 * h, e = sl < plan.n_routed ? plan.eid[sl] : -2;  // (-1: an entry without expert)
+      bool mine = p.m == 1 && e >= 0;  // (one token selects every slot)
+      if (p.m > 1)
+        for (int k = 0; k < p.top_k; ++k) mine |= s_cand[t * p.top_k + k] == e;
+      sel[h] = __ballot(mine);
+    }
+    float v = sum_slots_agent(p.part + o, stride, sel);
+    if (p.shared) v = __fadd_rn(v, sv);
     if (p.out_f32) p.out_f32[o] = v;
     if (p.out_bf16) p.out_bf16[o] = (uint16_t)f32_to_bf16_bits(v);
   }

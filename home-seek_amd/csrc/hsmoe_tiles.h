@@ -390,18 +390,27 @@ __device__ __forceinline__ unsigned add_agent(unsigned* p, unsigned v) {
   return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Fixed-order sum over the slots s < n with use[s] of agent-scope values
-// base[s * stride]: the loads go out 8 at a time so a chain of them costs one
-// memory round trip per 8 slots, and the additions keep slot order.
-__device__ __forceinline__ float sum_slots_agent(const float* base, int64_t stride, int n, const bool* use) {
+// Fixed-order sum of the agent-scope values base[s * stride] over the slots s
+// whose bit is set in sel (wave-uniform; slot s: bit s % 64 of word s / 64):
+// the loads go out 8 at a time so a chain of them costs one memory round trip
+// per 8 slots, and the additions keep slot order.
+__device__ __forceinline__ float sum_slots_agent(const float* base, int64_t stride, const uint64_t (&sel)[2]) {
   float v = 0.0f;
-  for (int s0 = 0; s0 < n; s0 += 8) {
-    float pv[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) pv[j] = (s0 + j < n) ? load_agent(base + (int64_t)(s0 + j) * stride) : 0.0f;
+  for (int h = 0; h < 2; ++h) {
+    uint64_t left = sel[h];
+    while (left) {
+      float pv[8];
+      const int n = __popcll(left);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (s0 + j < n && use[s0 + j]) v = __fadd_rn(v, pv[j]);
+      for (int j = 0; j < 8; ++j) {
+        pv[j] = j < n ? load_agent(base + (int64_t)(64 * h + __ffsll((unsigned long long)left) - 1) * stride) : 0.0f;
+        left &= left - 1;  // (0 stays 0)
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (j < n) v = __fadd_rn(v, pv[j]);
+    }
   }
   return v;
 }
