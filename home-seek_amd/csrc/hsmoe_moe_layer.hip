@@ -219,7 +219,7 @@ struct PlanBuild {
   alignas(4) unsigned char valid[kMaxExperts];  // expert e has a table entry
   alignas(4) unsigned char used[kMaxExperts];   // expert e is selected by some token
   short rank[kMaxExperts];                      // slot of a selected expert
-  unsigned char pslot[kMaxSlots];               // slot of top-k entry j (0xff: none, or an id met before)
+  unsigned tslots[kMaxTok][kMaxSlots / 32];     // slots of token t
 };
 
 // The slot plan lists the (slot, token) pairs the routing selects, slots
@@ -344,13 +344,18 @@ __device__ __forceinline__ void finish_plan(const LayerParams& p, Shared& sh, co
     if (b2) sh.b.rank[e4 + 2] = (short)(pre + b0 + b1);
     if (b3) sh.b.rank[e4 + 3] = (short)(pre + b0 + b1 + b2);
     reinterpret_cast<uint16_t*>(sh.tmask)[lane] = 0;  // all kMaxSlots == 128 bytes
+    static_assert(kMaxTok * kMaxSlots / 32 <= 64, "a lane per word");
+    if (lane < kMaxTok * kMaxSlots / 32) sh.b.tslots[lane / (kMaxSlots / 32)][lane % (kMaxSlots / 32)] = 0u;
     if (lane < kMaxTok) sh.ntp[lane] = 0;
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     // the pairs of top-k entries lane and lane + 64 (n <= kMaxSlots): slot
     // (-1: none) and weight.  Router ids are distinct per token; given ids may
-    // repeat, then the first carries the weights' sum in k order.
+    // repeat, which the second one's bit already set in the slot's mask shows
+    // (then, and only then, every entry looks at its token's ids one by one:
+    // done for every given route those loops cost 0.4 to 1.1 us at one token).
     int sl[2];
     float wt[2];
+    bool again = false;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int j = lane + 64 * h;
@@ -358,35 +363,38 @@ __device__ __forceinline__ void finish_plan(const LayerParams& p, Shared& sh, co
       wt[h] = 0.0f;
       if (j < n) {
         const int64_t e = sh.b.idx[j];
-        bool first = e >= 0 && e < p.n_exp && sh.b.valid[e];
-        if (!p.route_idx) {
+        if (e >= 0 && e < p.n_exp && sh.b.valid[e]) {
+          const int t = p.m == 1 ? 0 : j / p.top_k;
+          sl[h] = sh.b.rank[e];
           wt[h] = __fadd_rn(0.0f, sh.b.w[j]);
-        } else {
-          const int c0 = j / p.top_k * p.top_k;
-          for (int c = c0; c < j && first; ++c) first = sh.b.idx[c] != e;
-          if (first)
-            for (int c = c0; c < c0 + p.top_k; ++c)
-              if (sh.b.idx[c] == e) wt[h] = __fadd_rn(wt[h], sh.b.w[c]);
+          const unsigned bit = 1u << (8 * (sl[h] & 3) + t);
+          again |= (atomicOr(reinterpret_cast<unsigned*>(sh.tmask) + (sl[h] >> 2), bit) & bit) != 0;
+          if (p.m > 1) atomicOr(&sh.b.tslots[t][sl[h] >> 5], 1u << (sl[h] & 31));
         }
-        if (first) sl[h] = sh.b.rank[e];
+      }
+    }
+    if (__ballot(again) != 0) {  // an id met before in its token: the first one carries the weights' sum in k order
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (sl[h] < 0) continue;
+        const int j = lane + 64 * h, c0 = j / p.top_k * p.top_k;
+        const int64_t e = sh.b.idx[j];
+        bool first = true;
+        for (int c = c0; c < j && first; ++c) first = sh.b.idx[c] != e;
+        wt[h] = 0.0f;
+        for (int c = c0; c < c0 + p.top_k; ++c)
+          if (sh.b.idx[c] == e) wt[h] = __fadd_rn(wt[h], sh.b.w[c]);
+        if (!first) sl[h] = -1;
       }
     }
     if (p.m == 1) {  // one token: pair u is slot u
       if (sl[0] >= 0) {
-        sh.tmask[sl[0]] = 1;
         sh.ptok[sl[0]] = 0;
         sh.off[sl[0]] = sh.tpair[0][sl[0]] = (unsigned char)sl[0];
         sh.pw[sl[0]] = wt[0];
       }
       if (lane == 0) sh.ntp[0] = (unsigned char)base;
     } else {
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int j = lane + 64 * h;
-        if (j < n) sh.b.pslot[j] = (unsigned char)sl[h];
-        if (sl[h] >= 0)
-          atomicOr(reinterpret_cast<unsigned*>(sh.tmask) + (sl[h] >> 2), 1u << (8 * (sl[h] & 3) + j / p.top_k));
-      }
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       // first pairs: lane l counts slots 2l and 2l + 1 (at most 16 pairs), the
       // exclusive prefix of the counts from five ballots
@@ -404,15 +412,16 @@ __device__ __forceinline__ void finish_plan(const LayerParams& p, Shared& sh, co
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         if (sl[h] < 0) continue;
-        const int j = lane + 64 * h, t = j / p.top_k, c0 = t * p.top_k;
+        const int t = (lane + 64 * h) / p.top_k;
         const int u = sh.off[sl[h]] + __popc(sh.tmask[sl[h]] & ((1u << t) - 1u));
         sh.pw[u] = wt[h];
         sh.ptok[u] = (unsigned char)t;
         int r = 0, cnt = 0;  // among the token's slots
-        for (int c = c0; c < c0 + p.top_k; ++c) {
-          const int o = sh.b.pslot[c];
-          cnt += o != 0xff;
-          r += o < sl[h];
+#pragma unroll
+        for (int q = 0; q < kMaxSlots / 32; ++q) {
+          const unsigned w = sh.b.tslots[t][q];
+          cnt += __popc(w);
+          if (32 * q < sl[h]) r += __popc(sl[h] >= 32 * (q + 1) ? w : w & ((1u << (sl[h] & 31)) - 1u));
         }
         sh.tpair[t][r] = (unsigned char)u;
         if (r == 0) sh.ntp[t] = (unsigned char)cnt;

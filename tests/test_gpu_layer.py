@@ -364,3 +364,22 @@ def test_expert_that_is_not_finite_reaches_only_its_tokens(layer, dev):
     ops.moe_decode(x, idx, w, table, ops.SCALE_E8M0, None, 10.0, out_f32=b, d=D, i=I)
     for got in (a, b):
         assert torch.isnan(got[[0, 2]]).all() and torch.isfinite(got[1]).all()
+
+
+@pytest.mark.parametrize("m,ids", [(1, [3, 9, 3, -1, 300, 3]), (1, [5] * 16), (2, [7, 7, 2, 2, 7, 250]),
+                                   (8, [200, 131, 130, 200, 129, 128, 0, 131])])
+def test_given_ids_that_repeat(layer, dev, m, ids):
+    """A token's repeated ids are one pair with the weights' sum, whichever of the two plan loops the call takes."""
+    store, _, _ = layer
+    k = len(ids)
+    idx = torch.stack([torch.roll(torch.tensor(ids), t) for t in range(m)]).to(dev)
+    if m > 1:
+        idx[0] = torch.arange(k, device=dev) * 3  # a token without repeats beside them
+    w = torch.rand(m, k, device=dev, generator=torch.Generator(dev).manual_seed(6)) + 0.1
+    x = synthetic.hidden(SEED, 42, m, D, dev)
+    got = routed(x, idx, store.table(0), store.shared_entry(0), w=w, k=k)
+    f32 = torch.empty(m, D, dtype=torch.float32, device=dev)
+    ops.moe_decode(x, idx, w, store.table(0), ops.SCALE_E8M0, store.shared_entry(0), 10.0, out_f32=f32, d=D, i=I)
+    torch.cuda.synchronize()
+    assert ops.moe_layer_status(dev) == 0
+    assert torch.equal(got[1], f32)
