@@ -239,7 +239,6 @@ struct Shared {
   float pw[kMaxSlots];                             // weight of pair u
   alignas(4) unsigned char tmask[kMaxSlots];       // bit t: token t selects slot s
   unsigned char off[kMaxSlots];                    // first pair of slot s
-  unsigned char ptok[kMaxSlots];                   // token of pair u
   unsigned char tpair[kMaxTok][16];                // pairs of token t, slots ascending
   unsigned char ntp[kMaxTok];                      // how many
   unsigned tag;  // this launch's tag (read_launch_tag, once per workgroup)
@@ -313,8 +312,8 @@ __device__ __forceinline__ void build_plan_scores(const LayerParams& p, Shared& 
   }
 }
 
-// Slots from sh.b.idx / sh.w: the distinct valid ids ascending, each token's
-// weight of each slot, the slots' table entries.
+// Slots from sh.b.idx / sh.b.w: the distinct valid ids ascending, the (slot,
+// token) pairs with their weights, the slots' table entries.
 __device__ __forceinline__ void finish_plan(const LayerParams& p, Shared& sh, const uint64_t (&my_ent)[6]) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int n = p.m * p.top_k;
@@ -389,7 +388,6 @@ __device__ __forceinline__ void finish_plan(const LayerParams& p, Shared& sh, co
     }
     if (p.m == 1) {  // one token: pair u is slot u
       if (sl[0] >= 0) {
-        sh.ptok[sl[0]] = 0;
         sh.off[sl[0]] = sh.tpair[0][sl[0]] = (unsigned char)sl[0];
         sh.pw[sl[0]] = wt[0];
       }
@@ -415,7 +413,6 @@ __device__ __forceinline__ void finish_plan(const LayerParams& p, Shared& sh, co
         const int t = (lane + 64 * h) / p.top_k;
         const int u = sh.off[sl[h]] + __popc(sh.tmask[sl[h]] & ((1u << t) - 1u));
         sh.pw[u] = wt[h];
-        sh.ptok[u] = (unsigned char)t;
         int r = 0, cnt = 0;  // among the token's slots
 #pragma unroll
         for (int q = 0; q < kMaxSlots / 32; ++q) {
@@ -444,9 +441,9 @@ __device__ __forceinline__ void finish_plan(const LayerParams& p, Shared& sh, co
 // expert e's table entry.  The ids and weights come from the router's scores
 // (build_plan_scores) or, with given routing, from the caller's arrays (a
 // hash layer's token table, engine.py:1018-1023); then the distinct valid
-// expert ids in ascending order become the slots, each token's weight for a
-// slot being its weight for that id (a token's ids are distinct: at most
-// one), else 0 -- the union of _forward_legacy, fused_moe.py:466-476.
+// expert ids in ascending order become the slots (the union of
+// _forward_legacy, fused_moe.py:466-476), and each slot with each token that
+// selects it a pair, with the token's weight for that id.
 __device__ __forceinline__ void build_plan(const LayerParams& p, Shared& sh, const uint64_t (&my_ent)[6]) {
   const int n = p.m * p.top_k;
   if (p.route_idx) {
@@ -1251,8 +1248,11 @@ size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 size_t layer_lds(int64_t m, int64_t d, int64_t i) { return (size_t)(m * d > 2 * m * i ? m * d : 2 * m * i) * 2; }
 int64_t score_stride_words(int64_t m, int64_t n_exp) { return (m * n_exp * 8 + 4095) / 4096 * 512; }
 size_t scores_bytes(int64_t m, int64_t n_exp) { return (size_t)kScoreCopies * score_stride_words(m, n_exp) * 8; }
+// A launch uses m * top_k + 2 m rows of act (the pairs' activations, the shared
+// gate sums and activations) and of part (the pairs' partials, the shared ones,
+// the output rows fin).  The sizes leave a row for every (slot, token): callers
+// have allocated that much, and the no-alloc entry's limit on m follows from it.
 size_t act_bytes(int64_t m, int64_t i, int top_k) { return align256((size_t)(m * top_k + 2) * m * i * 8); }
-// partials of the m * top_k routed slots and the shared one, then the output rows (fin)
 size_t part_bytes(int64_t m, int64_t d, int top_k) { return align256((size_t)(m * top_k + 2) * m * d * 8); }
 
 // Workgroups of moe_layer_kernel the device holds at once, for an LDS size.
