@@ -216,10 +216,14 @@ extern "C" int hsmoe_router_topk(const void* x, const void* gate_w, const float*
       launch((const uint16_t*)x, (const uint16_t*)gate_w, bias, m, d, n_experts, top_k, scaling,
              (uint16_t*)logits_out, stage, counters, idx_out, w_out, (hipStream_t)stream);
     };
-    // one 16 x 16 tile per workgroup while that leaves CUs idle otherwise
-    // (m = 256 / 509 / 1024: 23 / 41 / 79 us, against 51 / 53 / 54 with the
-    // 32 x 32 tiles, which convert half as many operands per product)
-    if (m <= 640) go(launch_mfma<1, 8>);
+    // 16 x 16 tiles below 2.5 of them per CU; from there on 32 x 32 ones, which
+    // convert half as many operands per product but take 2.5 times as long each
+    // and leave CUs without one.  us with 16 / 32, d = 4096: 256 experts and
+    // m = 256 / 509 / 640 / 700 / 1024: 23 / 51, 41 / 53, 54 / 53, 57 / 53,
+    // 77 / 53; 64 experts and m = 800 / 2000 / 2700 / 4096: 19 / 48, 38 / 50,
+    // 55 / 50, 72 / 50; 8 experts and m = 4096: 20 / 48 (the FMA form 63).
+    const int64_t tiles = (n_experts + 15) / 16 * ((m + 15) / 16);
+    if (2 * tiles < 5 * device_cus()) go(launch_mfma<1, 8>);
     else go(launch_mfma<2, 8>);
     return check_launch("hsmoe_router_topk");
   }

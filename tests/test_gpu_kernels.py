@@ -104,6 +104,20 @@ def test_router_many_tokens_bit_exact(dev, m, n_exp, d, k):
         np.testing.assert_allclose(w.cpu().numpy(), rw, rtol=2e-6, atol=0)
 
 
+# 640 tiles of 16 x 16 are 2.5 per CU of 256: from there on the 32 x 32 ones; either side, ragged ends of both
+@pytest.mark.parametrize("m,n_exp,d,k", [(1009, 160, 512, 6), (1008, 160, 1024, 6), (177, 1000, 512, 8),
+                                         (161, 999, 512, 16), (641, 250, 2048, 6), (4081, 33, 512, 6)])
+def test_router_tile_choice_bit_exact(dev, m, n_exp, d, k):
+    gate, bias = synthetic.router_weights(m, 0, n_exp, d, dev)
+    x = synthetic.hidden(m, 0, m, d, dev)
+    idx, w, lg = ops.router_topk(x, gate, bias, k, 1.5, want_logits=True)
+    ridx, rw, _, rlg = orc.router(orc.to_np_bf16(x), orc.to_np_bf16(gate), bias.cpu().numpy(), k, 1.5,
+                                  return_scores=True)
+    assert np.array_equal(orc.to_np_bf16(lg), rlg)
+    assert np.array_equal(idx.cpu().numpy(), ridx)
+    np.testing.assert_allclose(w.cpu().numpy(), rw, rtol=2e-6, atol=0)
+
+
 def test_router_ties_and_no_bias(dev):
     x = torch.ones(2, 512, dtype=torch.bfloat16, device=dev)
     gate = torch.full((64, 512), 0.5, dtype=torch.bfloat16, device=dev)
