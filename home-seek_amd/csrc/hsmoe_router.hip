@@ -3,13 +3,12 @@
 // Restates compute_expert_affinity_with_bias (router.py:22-36).
 //
 // One launch in one of two forms:
-//  - m <= 8: a wave per expert row sums the chunk's tokens one after the other
-//    in fp64 FMAs (router_kernel; latency bound, the 2 MiB gate matrix is read
-//    once);
+//  - m <= 8: a wave per expert row sums the tokens one after the other in fp64
+//    FMAs (router_kernel; latency bound, the 2 MiB gate matrix is read once);
 //  - m > 8: tiles of tokens x experts on v_mfma_f64_16x16x4_f64
 //    (router_mfma_kernel).
-// In both, the last block of a token chunk to finish selects the top-k of each
-// of its tokens with (score desc, index asc) order == torch.sort(stable=True).
+// In both, the last block of the tokens (of a tile's tokens) to finish selects
+// the top-k of each of them with (score desc, index asc) order == torch.sort(stable=True).
 #include <math.h>
 
 #include "hsmoe_common.h"
@@ -21,43 +20,40 @@ namespace {
 
 constexpr int kTok = kRouterTok;
 constexpr int kLogitWaves = 4;  // expert rows per logits workgroup
-constexpr size_t kCounterBytes = 4096;
+constexpr size_t kCounterBytes = 4096;  // arrival counters: one per 16 or 32 tokens
+constexpr int64_t kMaxRows = 8192;
+static_assert(kMaxRows / 16 * 4 <= kCounterBytes, "a counter per tile of tokens");
 
-// Block (expert group bx, token chunk by): wave w computes the logits of
-// expert 4*bx + w for the chunk's (<= 8) tokens -- lane l holds columns
-// 8l + 512c .. +8 of the row for every c, all loads issued before the math.
-// The last block of a chunk (agent-scope arrival counter) runs the top-k of
-// the chunk's tokens, one token per wave, and re-arms the counter.
+// m <= kTok tokens.  Block b: wave w computes the logits of expert 4b + w for
+// the tokens -- lane l holds columns 8l + 512c .. +8 of the row for every c,
+// all loads issued before the math.  The last block (agent-scope arrival
+// counter) runs the top-k of the tokens, one token per wave, and re-arms the
+// counter.
 __global__ void __launch_bounds__(64 * kLogitWaves)
     router_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias,
-                  int64_t m, int64_t d, int64_t n_exp, int top_k, float scaling, uint16_t* __restrict__ logits_out,
+                  int m, int64_t d, int64_t n_exp, int top_k, float scaling, uint16_t* __restrict__ logits_out,
                   float* __restrict__ stage, unsigned* __restrict__ counters, int64_t* __restrict__ idx_out,
                   float* __restrict__ w_out) {
-  extern __shared__ __align__(16) uint16_t xs[];  // [nt][d]
+  extern __shared__ __align__(16) uint16_t xs[];  // [m][d]
   __shared__ int s_last;
   const int wave = threadIdx.x >> 6;
   const int64_t e = (int64_t)blockIdx.x * kLogitWaves + wave;
-  const int64_t t0 = (int64_t)blockIdx.y * kTok;
-  const int nt = (int)((m - t0) < kTok ? (m - t0) : kTok);
   // the gate rows do not depend on x: issue their loads before staging x
   uint4 wv[kMaxChunks];
   if (e < n_exp) load_gate_row(w, e, d, wv);
-  for (int64_t q = threadIdx.x; q < nt * d / 8; q += blockDim.x)
-    reinterpret_cast<uint4*>(xs)[q] = reinterpret_cast<const uint4*>(x + t0 * d)[q];
+  for (int64_t q = threadIdx.x; q < m * d / 8; q += blockDim.x)
+    reinterpret_cast<uint4*>(xs)[q] = reinterpret_cast<const uint4*>(x)[q];
   __syncthreads();
-  if (e < n_exp)
-    router_row(wv, xs, nt, d, e, n_exp, bias, logits_out ? logits_out + t0 * n_exp + e : nullptr,
-               stage + t0 * n_exp + e);
+  if (e < n_exp) router_row(wv, xs, m, d, e, n_exp, bias, logits_out ? logits_out + e : nullptr, stage + e);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   if (threadIdx.x == 0)
-    s_last = __hip_atomic_fetch_add(&counters[blockIdx.y], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-             gridDim.x - 1;
+    s_last = __hip_atomic_fetch_add(counters, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
   __syncthreads();
   if (!s_last) return;
-  for (int t = wave; t < nt; t += kLogitWaves)
-    wave_topk(stage + (t0 + t) * n_exp, n_exp, top_k, scaling, idx_out + (t0 + t) * top_k, w_out + (t0 + t) * top_k);
-  if (threadIdx.x == 0) __hip_atomic_store(&counters[blockIdx.y], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int t = wave; t < m; t += kLogitWaves)
+    wave_topk(stage + t * n_exp, n_exp, top_k, scaling, idx_out + t * top_k, w_out + t * top_k);
+  if (threadIdx.x == 0) __hip_atomic_store(counters, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Tiles of 16 kT tokens x 16 kT experts on the fp64 matrix cores, the columns
@@ -203,8 +199,7 @@ extern "C" int hsmoe_router_topk(const void* x, const void* gate_w, const float*
   if (d % 512 != 0 || d > 8192 || !aligned(x, 16) || !aligned(gate_w, 16))
     return fail(HSMOE_ERR_SHAPE,
                 "hsmoe_router_topk: d must be a multiple of 512 (<= 8192) and x/gate_w 16-byte aligned");
-  const int64_t chunks = (m + kTok - 1) / kTok;
-  if ((size_t)chunks * 4 > kCounterBytes) return fail(HSMOE_ERR_SHAPE, "hsmoe_router_topk: m must be <= 8192");
+  if (m > kMaxRows) return fail(HSMOE_ERR_SHAPE, "hsmoe_router_topk: m must be <= %lld", (long long)kMaxRows);
   if (!workspace || workspace_bytes < hsmoe_router_workspace_size(m, n_experts) || !aligned(workspace, 256))
     return fail(HSMOE_ERR_WORKSPACE, "hsmoe_router_topk: zero-filled 256-byte aligned workspace of %zu bytes needed",
                 hsmoe_router_workspace_size(m, n_experts));
@@ -227,10 +222,10 @@ extern "C" int hsmoe_router_topk(const void* x, const void* gate_w, const float*
     else go(launch_mfma<2, 8>);
     return check_launch("hsmoe_router_topk");
   }
-  dim3 grid((unsigned)((n_experts + kLogitWaves - 1) / kLogitWaves), (unsigned)chunks);
-  const size_t lds = (size_t)(m < kTok ? m : kTok) * d * 2;
+  const dim3 grid((unsigned)((n_experts + kLogitWaves - 1) / kLogitWaves));
+  const size_t lds = (size_t)m * d * 2;
   hipLaunchKernelGGL(router_kernel, grid, dim3(64 * kLogitWaves), lds, (hipStream_t)stream, (const uint16_t*)x,
-                     (const uint16_t*)gate_w, bias, m, d, n_experts, top_k, scaling, (uint16_t*)logits_out, stage,
+                     (const uint16_t*)gate_w, bias, (int)m, d, n_experts, top_k, scaling, (uint16_t*)logits_out, stage,
                      counters, idx_out, w_out);
   return check_launch("hsmoe_router_topk");
 }
