@@ -48,7 +48,6 @@ namespace hsmoe {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kGroupThreads = 1024;  // group kernel: one workgroup per expert and CU
 constexpr int kChunk = 32;        // tokens per chunk (two 16-token MFMA tiles)
 constexpr int kBigChunk = 64;     // tokens per chunk of an expert with more than kChunk pairs
 constexpr int kGuRT = 1;          // 16-row tiles per wave, gate/up (W1 and W3)
@@ -130,6 +129,7 @@ __device__ __forceinline__ int block_sum(int v, int* s_red) {
 // expert's chunks come first in both lists: every token is in one of them, so
 // its workgroups are the fullest, and they run under the routed stream (as
 // launches of their own they took 25 MB of weights 60 + 40 us at m = 509).
+template <int kGroupThreads>
 __global__ void __launch_bounds__(kGroupThreads) prefill_group_kernel(PrefillParams p) {
   constexpr int kWaves = kGroupThreads / 64;
   __shared__ uint16_t s_e[kMaxPairs];  // expert of pair q, kNone: invalid id or absent expert
@@ -1125,7 +1125,12 @@ extern "C" int hsmoe_moe_prefill(const void* x, int64_t m, int64_t d, int64_t i,
   const int64_t Cd = p.wide ? C : p.n_sh_dn + max_routed_chunks(m, n_experts, top_k);
   const int64_t n_bigs = pk / (p.small + 1) < touched ? pk / (p.small + 1) : touched;
   const int64_t big = p.wide ? p.n_sh_gu + (pk / p.big_chunk + n_bigs + 7) / 8 * 8 : 0;
-  hipLaunchKernelGGL(prefill_group_kernel, dim3((unsigned)n_experts + 1), dim3(kGroupThreads), 0, st, p);
+  // 256 threads per expert up to four pairs each, then 1024 (starting 16 waves
+  // costs what they save before): us with 256 / 1024, 64 experts and 54, 600,
+  // 1200, 1800, 12288 pairs 4.1 / 5.0, 5.2 / 5.4, 6.1 / 5.8, 7.8 / 6.1, 27 / 13;
+  // one expert and 36, 600, 1200, 1800 3.3 / 4.2, 4.4 / 5.0, 5.8 / 5.8, 8.9 / 8.0.
+  if (pk <= 1024) hipLaunchKernelGGL(prefill_group_kernel<256>, dim3((unsigned)n_experts + 1), dim3(256), 0, st, p);
+  else hipLaunchKernelGGL(prefill_group_kernel<1024>, dim3((unsigned)n_experts + 1), dim3(1024), 0, st, p);
   int rc = check_launch(name);
   if (rc) return rc;
   const dim3 blk(kThreads);

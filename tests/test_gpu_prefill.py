@@ -201,6 +201,23 @@ def test_full_shape_m512_zipf(dev):
     check_close(f32.cpu().numpy(), orc.to_np_bf16(out), dec.cpu().numpy(), "M=512 vs decode kernels")
 
 
+@pytest.mark.parametrize("m,k", [(128, 8), (205, 5), (129, 8), (511, 2), (513, 2)])
+def test_group_kernel_either_side_of_1024_pairs(small, dev, m, k):
+    """Up to 1024 pairs are grouped by 256 threads, more by 1024: rows as of calls of 64 tokens, bit for bit
+    (a pair's sums do not depend on its chunk)."""
+    x = synthetic.hidden(SEED, 60 + m, m, small.d, dev)
+    g = torch.Generator(dev).manual_seed(m)
+    idx = torch.stack([torch.randperm(small.E + 2, generator=g, device=dev)[:k] - 1 for _ in range(m)])  # (-1, E: none)
+    w = torch.rand(m, k, device=dev, generator=g)
+    table, shared = small.store.table(0), small.store.shared_entry(0)
+    whole, parts = (torch.empty(m, small.d, dtype=torch.float32, device=dev) for _ in range(2))
+    ops.moe_prefill(x, idx, w, table, ops.SCALE_E8M0, shared, 10.0, out_f32=whole, i=small.i)
+    for a in range(0, m, 64):
+        ops.moe_prefill(x[a:a + 64], idx[a:a + 64], w[a:a + 64], table, ops.SCALE_E8M0, shared, 10.0,
+                        out_f32=parts[a:a + 64], i=small.i)
+    assert torch.equal(whole, parts)
+
+
 @pytest.fixture(scope="module")
 def odd(dev):
     m = Model(dev, 9, 1024, 1536)  # 6 K-chunks in the down pass: its last read of scales is a half one
