@@ -1111,14 +1111,20 @@ extern "C" int hsmoe_moe_prefill(const void* x, int64_t m, int64_t d, int64_t i,
   // experts of 12, 16, 23, 32 and 47 pairs 844 / 867, 925 / 927, 1060 / 1018,
   // 1307 / 1195, 1640 / 1388; 64 experts of 28 pairs (two rounds of
   // workgroups) 319 / 358; one bf16 expert of 40, 500 and 4096 pairs 154 / 117,
-  // 170 / 122, 836 / 407.  One expert's chunks are of 32 pairs where those give
-  // at most one workgroup per CU (500 pairs: 122, of 64 pairs 151; 1024 pairs of
-  // 64 158, 1023 of 32 192).
+  // 170 / 122, 836 / 407.
   const bool one = n_experts == 1;
   p.wide = one ? pk > kChunk : pk >= 24 * n_experts && pk * i >= (int64_t)12288 * 1024;
   p.small = p.wide && one ? 0 : kChunk;
-  const int64_t blocks = i / kWideGuRows > d / kWideDnRows ? i / kWideGuRows : d / kWideDnRows;
-  p.big_chunk = p.wide && one && (pk + kChunk - 1) / kChunk * blocks <= 256 ? kChunk : kBigChunk;
+  // One expert's chunks are of 32 pairs where these give either pass at most one
+  // workgroup per CU, or one pass at most 3/4 of that (which 64-pair chunks would
+  // halve): us with 32 / 64, d = 4096, i = 2048, bf16, 500 and 700 pairs 85 / 99,
+  // 124 / 102; d = 1024, i = 2048, E8M0, 700, 1500 and 3000 pairs 44 / 55,
+  // 53 / 64, 88 / 83 (the small kernels 49, 62, 94), bf16 60 / 66, 74 / 80,
+  // 124 / 104.
+  const int64_t n32 = (pk + kChunk - 1) / kChunk, gu_blocks = n32 * (i / kWideGuRows), dn_blocks = n32 * (d / kWideDnRows);
+  const int64_t more = gu_blocks > dn_blocks ? gu_blocks : dn_blocks, fewer = gu_blocks + dn_blocks - more;
+  const bool few = more <= device_cus() || 4 * fewer <= 3 * device_cus();
+  p.big_chunk = p.wide && one && few ? kChunk : kBigChunk;
   p.by_rows = n_experts < 8;
   // chunks of the small kernels (beside the wide ones at most one per expert), and of the wide ones
   const int64_t C = p.wide ? (p.small ? touched : 0) : p.n_sh_gu + max_routed_chunks(m, n_experts, top_k);
