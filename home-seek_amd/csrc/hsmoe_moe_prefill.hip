@@ -1104,16 +1104,19 @@ extern "C" int hsmoe_moe_prefill(const void* x, int64_t m, int64_t d, int64_t i,
   p.n_sh_gu = shared ? (int)((m + kBigChunk - 1) / kBigChunk) : 0;
   p.n_sh_dn = shared ? (int)((m + kChunk - 1) / kChunk) : 0;
   const int64_t pk = m * top_k, touched = n_experts < pk ? n_experts : pk;
-  // The wide kernels take calls of 24 pairs per expert and more whose chunks
-  // fill the chip about four times (two workgroups per CU, i / 128 or d / 256
-  // of them per chunk of ~48 pairs), and every call of one expert with more
-  // than a chunk of pairs.  Small / wide kernels, us, d = 4096, i = 2048: 256
+  // The wide kernels take calls of 24 pairs per expert and more (32 without the
+  // shared expert, whose 64-pair chunks gain most) whose chunks fill the chip
+  // about four times (two workgroups per CU, i / 128 or d / 256 of them per chunk
+  // of ~48 pairs), and every call of one expert with more than a chunk of pairs.
+  // Small / wide kernels, us, d = 4096, i = 2048, with the shared expert: 256
   // experts of 12, 16, 23, 32 and 47 pairs 844 / 867, 925 / 927, 1060 / 1018,
-  // 1307 / 1195, 1640 / 1388; 64 experts of 28 pairs (two rounds of
-  // workgroups) 319 / 358; one bf16 expert of 40, 500 and 4096 pairs 154 / 117,
-  // 170 / 122, 836 / 407.
+  // 1307 / 1195, 1640 / 1388; 64 experts of 28 pairs (two rounds of workgroups)
+  // 319 / 358.  Without it: 256 experts of 28, 31 and 38 pairs 973 / 1012,
+  // 1028 / 1031, 1143 / 1126 (d = 2048, fp32 scales 658 / 685, 702 / 698,
+  // 780 / 738).  One bf16 expert of 40, 500 and 4096 pairs 154 / 117, 170 / 122,
+  // 836 / 407.
   const bool one = n_experts == 1;
-  p.wide = one ? pk > kChunk : pk >= 24 * n_experts && pk * i >= (int64_t)12288 * 1024;
+  p.wide = one ? pk > kChunk : pk >= (shared ? 24 : 32) * n_experts && pk * i >= (int64_t)12288 * 1024;
   p.small = p.wide && one ? 0 : kChunk;
   // One expert's chunks are of 32 pairs where these give either pass at most one
   // workgroup per CU, or one pass at most 3/4 of that (which 64-pair chunks would
