@@ -48,11 +48,13 @@ def test_layer_kernel_no_scratch_two_waves_per_simd(tmp_path):
 
 @pytest.mark.skipif(shutil.which("/opt/rocm/bin/hipcc") is None, reason="hipcc not present")
 def test_prefill_kernels_no_scratch(tmp_path):
-    """Every instantiation of the prefill gate/up and down kernels (FP4 at 4
-    waves per SIMD for gate/up, FP8 and bf16 for the shared expert) keeps its
-    registers: a spill would slow prefill with no test noticing."""
+    """Every instantiation of the prefill gate/up, down and wide kernels (four,
+    three and two waves per SIMD; the wide ones take all 256 registers) keeps
+    its registers: a spill would slow prefill with no test noticing."""
     found = _resources("hsmoe_moe_prefill.hip", tmp_path)
-    kern = {n: v for n, v in found.items() if "prefill_gate_up_kernel" in n or "prefill_down_kernel" in n}
-    assert any("prefill_gate_up_kernel" in n for n in kern) and any("prefill_down_kernel" in n for n in kern), list(found)
+    kinds = ("prefill_gate_up_kernel", "prefill_down_kernel", "prefill_wide_kernel")
+    kern = {n: v for n, v in found.items() if any(k in n for k in kinds)}
+    for k in kinds:
+        assert any(k in n for n in kern), (k, list(found))
     bad = {n: v for n, v in kern.items() if v[0] != 0}
     assert not bad, f"prefill kernels with scratch: {bad}"

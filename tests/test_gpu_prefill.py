@@ -225,23 +225,35 @@ def odd(dev):
     return m
 
 
-@pytest.mark.parametrize("kind", ["e8m0", "f32", "bf16"])
-@pytest.mark.parametrize("n_exp,m,shared", [(1, 33, False), (1, 500, False), (1, 1089, True), (2, 40, True),
-                                            (9, 131, True)])
-def test_wide_kernels_every_format(odd, dev, kind, n_exp, m, shared):
-    """Calls whose experts hold many pairs (the 32-row kernels): every weight format, chunks of one and two
-    32-pair tiles with ragged ends, one expert (chunks of 32 below 1024 pairs, else 64), chunks placed by row
-    block (fewer than 8 experts) or by chunk, small experts beside big ones (ids 7 and 8 of 9)."""
-    k = 1 if n_exp < 3 else 2
+def wide_rule(pairs, n_exp, i, shared):
+    """Which calls take the 32-row kernels (hsmoe_moe_prefill's rule)."""
+    return pairs > 32 if n_exp == 1 else pairs >= (24 if shared else 32) * n_exp and pairs * i >= 12288 * 1024
+
+
+def entries_of(model, n_exp, kind):
+    """The first n_exp experts in one of the weight formats."""
     entries = []
     for e in range(n_exp):
-        w1, s1, w3, s3, w2, s2 = odd.store.expert_views(0, e)
+        w1, s1, w3, s3, w2, s2 = model.store.expert_views(0, e)
         if kind == "bf16":
             entries.append(tuple(ops.fp4_dequant_bf16(a, b) for a, b in ((w1, s1), (w3, s3), (w2, s2))))
         elif kind == "f32":
             entries.append((w1, s1.to(torch.float32), w3, s3.to(torch.float32), w2, s2.to(torch.float32)))
         else:
             entries.append((w1, s1, w3, s3, w2, s2))
+    return entries
+
+
+@pytest.mark.parametrize("kind", ["e8m0", "f32", "bf16"])
+@pytest.mark.parametrize("n_exp,m,shared", [(1, 33, False), (1, 500, False), (1, 1089, True), (1, 1601, False),
+                                            (2, 40, True), (9, 131, True)])
+def test_wide_kernels_every_format(odd, dev, kind, n_exp, m, shared):
+    """One expert on the 32-row kernels in every weight format: chunks of 32 pairs (33, 500 and 1089) and of 64
+    (1601, the shared expert's) with ragged ends.  The calls of 2 and 9 experts are below the line of those
+    kernels (wide_rule): the same formats on the 16-row ones."""
+    assert wide_rule(m * (1 if n_exp < 3 else 2), n_exp, odd.i, shared) == (n_exp == 1)
+    k = 1 if n_exp < 3 else 2
+    entries = entries_of(odd, n_exp, kind)
     table = ops.expert_table(entries, dev)
     x = synthetic.hidden(SEED, 40 + m, m, odd.d, dev)
     idx = np.stack([(np.arange(m) * (j + 1) + j) % min(n_exp, 7) for j in range(k)], axis=1).astype(np.int64)
@@ -257,3 +269,52 @@ def test_wide_kernels_every_format(odd, dev, kind, n_exp, m, shared):
     sample = np.unique(np.r_[0:m:7, 30:34, m - 3:m] % m)
     ref = odd.oracle(x[sample], idx[sample], w[sample], shared=shared)
     check_close(f32[sample].cpu().numpy(), orc.to_np_bf16(out[sample]), ref, f"wide {kind} E={n_exp} m={m}")
+
+
+@pytest.mark.parametrize("kind", ["e8m0", "f32", "bf16"])
+@pytest.mark.parametrize("n_exp,m,shared", [(9, 4099, True), (9, 4099, False), (7, 4107, True), (2, 4098, False)])
+def test_wide_kernels_several_experts(odd, dev, kind, n_exp, m, shared):
+    """The 32-row kernels in calls of several experts: chunks placed by chunk (9 experts) and by row block (7 and 2),
+    small experts beside them (5 and 32 pairs: the 16-row kernels), chunks of 33, 64 and 64 + 1 pairs and long ones,
+    an absent expert, invalid ids, the shared expert's FP8 chunks before the routed ones."""
+    k = 2
+    assert wide_rule(m * k, n_exp, odd.i, shared)
+    entries = entries_of(odd, n_exp, kind)
+    idx = np.stack([np.arange(m) % 2, np.full(m, -1)], axis=1).astype(np.int64)
+    few = 0  # tokens below this select experts of at most 32 pairs only
+    if n_exp > 2:
+        entries[3] = None
+        counts = {4: 5, 5: 32, 6: 33} if n_exp == 7 else {4: 5, 5: 32, 6: 33, 7: 64, 8: 65}
+        few = counts[4] + counts[5]
+        idx[:few, 0], idx[:few, 1] = np.repeat([4, 5], [5, 32]), [-1, n_exp, 3] * 12 + [-1]
+        at = few
+        for e in sorted(counts)[2:]:
+            idx[at:at + counts[e], 1] = e
+            at += counts[e]
+        idx[at:at + 2000, 1] = 2
+        assert np.bincount(idx[idx >= 0], minlength=n_exp)[4:n_exp].tolist() == list(counts.values())
+    else:
+        idx[:, 1] = 1 - idx[:, 0]
+        idx[::5, 1] = 2  # (no such expert)
+    w = np.linspace(0.2, 1.1, m * k, dtype=np.float32).reshape(m, k)
+    table, scale = ops.expert_table(entries, dev), ops.SCALE_F32 if kind == "f32" else ops.SCALE_E8M0
+    sh = odd.store.shared_entry(0) if shared else None
+    x = synthetic.hidden(SEED, 70 + m, m, odd.d, dev)
+    ti, tw = torch.as_tensor(idx, device=dev), torch.as_tensor(w, device=dev)
+    whole, parts = (torch.empty(m, odd.d, dtype=torch.float32, device=dev) for _ in range(2))
+    out, _ = ops.moe_prefill(x, ti, tw, table, scale, sh, 10.0, out_f32=whole, i=odd.i)
+    for a in range(0, m, 512):  # below the line: the 16-row kernels
+        assert not wide_rule(512 * k, n_exp, odd.i, shared)
+        ops.moe_prefill(x[a:a + 512], ti[a:a + 512], tw[a:a + 512], table, scale, sh, 10.0,
+                        out_f32=parts[a:a + 512], i=odd.i)
+    # the two forms add in another order, and the small experts' pairs keep the 16-row one
+    assert not torch.equal(whole[few:], parts[few:])
+    if not shared:
+        assert torch.equal(whole[:few], parts[:few])
+    what = f"wide {kind} E={n_exp} m={m} shared={shared}"
+    check_close(whole.cpu().numpy(), orc.to_np_bf16(out), parts.cpu().numpy(), what + " vs 16-row kernels")
+    sample = np.unique(np.r_[0:few:6, few:few + 300:11, m - 3:m] % m)
+    taken = idx[sample].copy()
+    taken[(taken >= n_exp) | ((taken == 3) & (n_exp > 2))] = -1
+    check_close(whole[sample].cpu().numpy(), orc.to_np_bf16(out[sample]),
+                odd.oracle(x[sample], taken, w[sample], shared=shared), what)
