@@ -55,7 +55,7 @@ def _copied(w: tuple, dev: torch.device) -> bool:
 
 
 def _fp4_entry(w: tuple, dev: torch.device):
-    """Normalises a reference 6-tuple; returns (entry tuple, scale_kind, _copied).
+    """Normalises a reference 6-tuple; returns (entry tuple, scale_kind).
 
     A tuple that needs nothing (contiguous on the device, E8M0 or fp32 scales)
     is taken as it is: a call of FusedMoEFFN.forward makes one entry per
@@ -63,8 +63,7 @@ def _fp4_entry(w: tuple, dev: torch.device):
     if (len(w) == 6 and w[0].dtype in _FP4_DTYPES and w[2].dtype in _FP4_DTYPES and w[4].dtype in _FP4_DTYPES
             and w[1].dtype in _SCALE_KINDS and w[3].dtype == w[1].dtype and w[5].dtype == w[1].dtype
             and _ready(w, dev)):
-        return tuple(w), _SCALE_KINDS[w[1].dtype], False
-    copied = _copied(w, dev)
+        return tuple(w), _SCALE_KINDS[w[1].dtype]
     w1, s1, w3, s3, w2, s2 = (_as_device(t, dev) for t in w)
     kinds = set()
     out = []
@@ -76,12 +75,11 @@ def _fp4_entry(w: tuple, dev: torch.device):
         out += [data.contiguous(), sc2.contiguous()]
     if len(kinds) != 1:
         raise TypeError("all three scales of one expert must share one dtype")
-    return tuple(out), kinds.pop(), copied
+    return tuple(out), kinds.pop()
 
 
 def _bf16_entry(w: tuple, dev: torch.device):
-    """A reference 3-tuple as bf16 on the device; returns (entry tuple, _copied)."""
-    return tuple(_as_device(t, dev).to(torch.bfloat16).contiguous() for t in w), _copied(w, dev)
+    return tuple(_as_device(t, dev).to(torch.bfloat16).contiguous() for t in w)
 
 
 def _run_decode_chunks(x: torch.Tensor, topk_idx: torch.Tensor, topk_w: torch.Tensor, table: torch.Tensor,
@@ -150,15 +148,16 @@ class FusedMoEFFN:
             if w is None:
                 continue
             if len(w) == 6:
-                ent, kind, copied = _fp4_entry(w, dev)
+                ent, kind = _fp4_entry(w, dev)
                 kinds.add(kind)
                 inter = ent[0].shape[0]
             elif len(w) == 3:
-                ent, copied = _bf16_entry(w, dev)
+                ent = _bf16_entry(w, dev)
                 inter = ent[0].shape[0]
             else:
                 continue
-            wait = wait or copied
+            if ent is not w:  # (a ready entry is the loader's own)
+                wait = wait or _copied(w, dev)
             entries[eid] = ent
         if inter is None:
             return torch.zeros_like(hidden_states)
@@ -183,10 +182,10 @@ class FusedMoEFFN:
         kinds = set()
         wait = False
         for e in eids:
-            ent, kind, copied = _fp4_entry(fp4_data[e], dev)
+            ent, kind = _fp4_entry(fp4_data[e], dev)
             entries.append(ent)
             kinds.add(kind)
-            wait = wait or copied
+            wait = wait or _copied(fp4_data[e], dev)
         if len(kinds) > 1:
             raise TypeError("experts of one call mix E8M0 and fp32 scales")
         table = ops.expert_table(entries, dev, wait=wait)
@@ -239,7 +238,8 @@ def fused_expert_ffn_pt(hidden: torch.Tensor, w1: torch.Tensor, w3: torch.Tensor
                         swiglu_limit: float = 10.0) -> torch.Tensor:
     """One bf16 expert (fused_moe.py:383-395) as a weight-1 slot of the HIP FFN."""
     dev = hidden.device
-    (w1, w3, w2), copied = _bf16_entry((w1, w3, w2), dev)
+    copied = _copied((w1, w3, w2), dev)
+    w1, w3, w2 = _bf16_entry((w1, w3, w2), dev)
     table = ops.expert_table([(w1, w3, w2)], dev, wait=copied)
     m = hidden.shape[0]
     idx = torch.zeros(m, 1, dtype=torch.int64, device=dev)
@@ -257,12 +257,13 @@ def fused_expert_ffn_triton(hidden: torch.Tensor, w1: torch.Tensor, w3: torch.Te
     if w1.dtype in (torch.int8, torch.uint8):
         if w1_scale is None or w3_scale is None or w2_scale is None:
             raise ValueError("FP4 weights need all three scales")
-        ent, kind, copied = _fp4_entry((w1, w1_scale, w3, w3_scale, w2, w2_scale), dev)
-        inter = ent[0].shape[0]
+        given = (w1, w1_scale, w3, w3_scale, w2, w2_scale)
+        ent, kind = _fp4_entry(given, dev)
     else:
-        (ent, copied), kind = _bf16_entry((w1, w3, w2), dev), SCALE_E8M0
-        inter = ent[0].shape[0]
-    table = ops.expert_table([ent], dev, wait=copied)
+        given = (w1, w3, w2)
+        ent, kind = _bf16_entry(given, dev), SCALE_E8M0
+    inter = ent[0].shape[0]
+    table = ops.expert_table([ent], dev, wait=_copied(given, dev))
     m = hidden.shape[0]
     idx = torch.zeros(m, 1, dtype=torch.int64, device=dev)
     w = torch.ones(m, 1, dtype=torch.float32, device=dev)

@@ -161,6 +161,14 @@ def router_topk(x: torch.Tensor, gate_w: torch.Tensor, bias: torch.Tensor | None
     return (idx, w, logits) if want_logits else (idx, w)
 
 
+def _capturing(device: torch.device) -> bool:
+    """Whether the stream that copies to `device`, current or not, is being captured."""
+    if device.index is None or device.index == torch.cuda.current_device():
+        return torch.cuda.is_current_stream_capturing()
+    with torch.cuda.device(device):
+        return torch.cuda.is_current_stream_capturing()
+
+
 def expert_table(entries: list, device: torch.device, wait: bool = True) -> torch.Tensor:
     """uint64 [n][6] device table from per-expert tuples.
 
@@ -187,9 +195,7 @@ def expert_table(entries: list, device: torch.device, wait: bool = True) -> torc
     # the copy is done).  A graph would read the host memory again when others
     # own it: refused under capture.
     if torch.device(device).type == "cuda":
-        with torch.cuda.device(device):  # the copy runs on this device's stream
-            capturing = torch.cuda.is_current_stream_capturing()
-        if capturing:
+        if _capturing(torch.device(device)):
             raise RuntimeError("an expert table is made from host memory: not under graph capture")
         if not wait:
             return rows.pin_memory().to(device, non_blocking=True)

@@ -22,6 +22,7 @@ def current(monkeypatch):
         now[0] = before
 
     monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: now[0])
     return now
 
 
