@@ -372,7 +372,9 @@ __device__ __forceinline__ void finish_plan(const LayerParams& p, Shared& sh, co
         }
       }
     }
-    if (__ballot(again) != 0) {  // an id met before in its token: the first one carries the weights' sum in k order
+    // an id met before in its token: the first one carries the weights' sum in k
+    // order (laid out after the rest: in its way it cost 0.15 us at one token)
+    if (__builtin_expect(__ballot(again) != 0, 0)) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         if (sl[h] < 0) continue;
