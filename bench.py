@@ -778,7 +778,7 @@ def main():
     args = parse()
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) > 1:
         print("bench.py measures one GPU: this build has no multi-GPU path "
-              "(expert-parallel sharding is described in DESIGN.md, not run). Use --gpus 1.", file=sys.stderr)
+              "(expert-parallel sharding is not implemented). Use --gpus 1.", file=sys.stderr)
         sys.exit(2)
     import torch
     __graft_entry__.package()

@@ -12,12 +12,13 @@
 // activation enters the down GEMM as a bf16 hi + lo pair (a = hi + lo + O(2^-17 a)),
 // which the 16-column MFMA absorbs for free when m <= 8.
 //
-// Launch structure (both HBM-bound; see the DESIGN notes in the repo):
+// Launch structure (both HBM-bound):
 //   phase 1  grid (i/16, slots)  4 waves: wave w streams 16 rows x d/4 columns
 //            of W1 and W3 of one expert; the 4 partials meet in LDS in fixed
 //            order; SwiGLU, routing weight and the hi/lo split happen there.
-//   phase 2  grid (d/16)  16 waves: wave w streams units (slot, 512 columns)
-//            w, w+16, ... of W2 for 16 output rows; fixed-order LDS reduction.
+//   phase 2  grid (d/64, slots)  4 waves: wave w streams 16 rows of W2 of one
+//            expert; the last workgroup of a group of 64 rows adds each
+//            token's slots in slot order.
 // "Slots" are the distinct selected experts in ascending id order (the union
 // of _forward_legacy, fused_moe.py:466-476) followed by the shared expert.
 // Every workgroup derives the slot plan itself from topk_idx, so no host sync

@@ -1,7 +1,7 @@
 // Routed-expert SwiGLU FFN for many tokens (prefill): a grouped GEMM over the
 // experts the tokens select, each expert's weights streamed from HBM once per
 // chunk of its tokens (gate/up: up to 32, or 64 for an expert with more than
-// 32; down: up to 32).
+// 32; down: up to 32, or 64 in the wide kernels).
 //
 // Restates FusedMoEFFN._forward_legacy at B > 8 and the FP4 grouped route of
 // fused_expert_ffn_triton (fused_moe.py:269-380, 458-551) plus the shared
