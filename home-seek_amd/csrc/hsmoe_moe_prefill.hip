@@ -1134,11 +1134,12 @@ extern "C" int hsmoe_moe_prefill(const void* x, int64_t m, int64_t d, int64_t i,
   const int64_t Cd = p.wide ? C : p.n_sh_dn + max_routed_chunks(m, n_experts, top_k);
   const int64_t n_bigs = pk / (p.small + 1) < touched ? pk / (p.small + 1) : touched;
   const int64_t big = p.wide ? p.n_sh_gu + (pk / p.big_chunk + n_bigs + 7) / 8 * 8 : 0;
-  // 256 threads per expert up to four pairs each, then 1024 (starting 16 waves
+  // 256 threads per expert up to three pairs each, then 1024 (starting 16 waves
   // costs what they save before): us with 256 / 1024, 64 experts and 54, 600,
   // 1200, 1800, 12288 pairs 4.1 / 5.0, 5.2 / 5.4, 6.1 / 5.8, 7.8 / 6.1, 27 / 13;
-  // one expert and 36, 600, 1200, 1800 3.3 / 4.2, 4.4 / 5.0, 5.8 / 5.8, 8.9 / 8.0.
-  if (pk <= 1024) hipLaunchKernelGGL(prefill_group_kernel<256>, dim3((unsigned)n_experts + 1), dim3(256), 0, st, p);
+  // one expert and 36, 600, 1200, 1800 3.3 / 4.2, 4.4 / 5.0, 5.8 / 5.8, 8.9 / 8.0
+  // (a call of 1008 pairs of 64 small experts 39.0 / 38.6).
+  if (pk <= 768) hipLaunchKernelGGL(prefill_group_kernel<256>, dim3((unsigned)n_experts + 1), dim3(256), 0, st, p);
   else hipLaunchKernelGGL(prefill_group_kernel<1024>, dim3((unsigned)n_experts + 1), dim3(1024), 0, st, p);
   int rc = check_launch(name);
   if (rc) return rc;

@@ -201,9 +201,9 @@ def test_full_shape_m512_zipf(dev):
     check_close(f32.cpu().numpy(), orc.to_np_bf16(out), dec.cpu().numpy(), "M=512 vs decode kernels")
 
 
-@pytest.mark.parametrize("m,k", [(128, 8), (205, 5), (129, 8), (511, 2), (513, 2)])
-def test_group_kernel_either_side_of_1024_pairs(small, dev, m, k):
-    """Up to 1024 pairs are grouped by 256 threads, more by 1024: rows as of calls of 64 tokens, bit for bit
+@pytest.mark.parametrize("m,k", [(96, 8), (97, 8), (128, 6), (153, 5), (154, 5), (513, 2)])
+def test_group_kernel_either_side_of_768_pairs(small, dev, m, k):
+    """Up to 768 pairs are grouped by 256 threads, more by 1024: rows as of calls of 64 tokens, bit for bit
     (a pair's sums do not depend on its chunk)."""
     x = synthetic.hidden(SEED, 60 + m, m, small.d, dev)
     g = torch.Generator(dev).manual_seed(m)
