@@ -102,7 +102,7 @@ __device__ __forceinline__ double bf16_elem(const uint4& q, int e) {
 template <int kC>
 constexpr int row_step() { return kC >= 5 ? 1 : kC >= 3 ? 2 : kC == 2 ? 4 : 8; }
 
-template <int kC>
+template <int kC, int kR>
 __global__ void __launch_bounds__(64 * kRowWaves)
     lm_head_row_kernel(const uint16_t* __restrict__ w, const uint16_t* __restrict__ hb, int64_t vocab,
                        const int64_t* __restrict__ ids, uint16_t* __restrict__ logits, int64_t* __restrict__ pred_out,
@@ -111,7 +111,6 @@ __global__ void __launch_bounds__(64 * kRowWaves)
   __shared__ int s_last;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   constexpr int kRowQ = 64 * kC;  // 16-byte chunks per row
-  constexpr int kR = row_step<kC>();
   double hv[kC][8];
 #pragma unroll
   for (int j = 0; j < kC; ++j) {
@@ -186,18 +185,28 @@ __global__ void __launch_bounds__(64 * kRowWaves)
   if (s_last && threadIdx.x == 0) accept_tail<1>(ids, pred_out, result_out, ws);
 }
 
-template <int kC>
-int launch_row(const uint16_t* w, const uint16_t* h, int64_t vocab, const int64_t* ids, uint16_t* logits,
+template <int kC, int kR>
+int launch_rows(const uint16_t* w, const uint16_t* h, int64_t vocab, const int64_t* ids, uint16_t* logits,
                int64_t* pred, int64_t* result, Workspace* ws, hipStream_t st) {
   // one workgroup of 4 waves per CU: 168-174 us over the 129,280 x 4096 head
   // against 179-180 with two per CU (320 or 384 workgroups, uneven over the
   // CUs: 185-205)
   const int64_t blocks = device_cus();
-  const int64_t need = (vocab + kRowWaves * row_step<kC>() - 1) / (kRowWaves * row_step<kC>());
+  const int64_t need = (vocab + kRowWaves * kR - 1) / (kRowWaves * kR);
   const unsigned nb = (unsigned)(need < blocks ? need : blocks);
-  hipLaunchKernelGGL((lm_head_row_kernel<kC>), dim3(nb), dim3(64 * kRowWaves), 0, st, w, h, vocab, ids, logits, pred,
-                     result, ws);
+  hipLaunchKernelGGL((lm_head_row_kernel<kC, kR>), dim3(nb), dim3(64 * kRowWaves), 0, st, w, h, vocab, ids, logits,
+                     pred, result, ws);
   return check_launch("hsmoe_lm_head_accept");
+}
+
+// A head of at most two rows per CU: a row per step (several leave most waves
+// without one): us with a row / several per step, d = 512 and 100, 500, 1000
+// rows 4.5 / 6.3, 5.4 / 6.8, 7.7 / 6.9; d = 2048 4.6 / 5.0, 5.7 / 5.5, 8.0 / 6.2.
+template <int kC>
+int launch_row(const uint16_t* w, const uint16_t* h, int64_t vocab, const int64_t* ids, uint16_t* logits,
+               int64_t* pred, int64_t* result, Workspace* ws, hipStream_t st) {
+  if (vocab <= 2 * device_cus()) return launch_rows<kC, 1>(w, h, vocab, ids, logits, pred, result, ws, st);
+  return launch_rows<kC, row_step<kC>()>(w, h, vocab, ids, logits, pred, result, ws, st);
 }
 
 // ------------------------------------------------------------- fp64 MFMA form

@@ -169,6 +169,18 @@ def test_lm_head_row_steps_bit_exact(dev, n_tok, vocab, d):
             assert np.array_equal(pred.cpu().numpy(), orc.bf16_to_f32(ref).argmax(axis=1))
 
 
+# one token: up to 512 rows (two per CU of 256) one row per step, more rows several
+@pytest.mark.parametrize("vocab,d", [(511, 512), (512, 1024), (513, 512), (517, 1024), (515, 1536), (514, 2048)])
+def test_lm_head_few_rows_bit_exact(dev, vocab, d):
+    h = synthetic.hidden(vocab, 1, 1, d, dev)
+    lm = synthetic.normal_bf16(vocab, 77, (vocab, d), 0.0, 0.02, dev)
+    ref = orc.logits_bf16(orc.to_np_bf16(h), orc.to_np_bf16(lm))
+    for _ in range(2):
+        logits, pred, _ = ops.lm_head_accept(h, lm, None)
+        assert np.array_equal(orc.to_np_bf16(logits), ref)
+        assert np.array_equal(pred.cpu().numpy(), orc.bf16_to_f32(ref).argmax(axis=1))
+
+
 def test_lm_head_accept_kats_on_device(dev):
     """The reference's accept/reject KATs (tests/test_mtp.py:355-456) with one-hot lm_head rows."""
     d, vocab = 512, 128
