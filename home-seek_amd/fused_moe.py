@@ -47,11 +47,14 @@ def _ready(w: tuple, dev: torch.device) -> bool:
     return True
 
 
-def _copied(w: tuple, dev: torch.device) -> bool:
-    """Some tensor of the entry comes from elsewhere (pinned host memory: its
-    copy may still be running when _as_device returns, and the caller may
-    refill the buffer once the call that uses it has returned)."""
-    return any(t.device != dev for t in w)
+def _copied(w: tuple, entry: tuple, dev: torch.device) -> bool:
+    """Some tensor of w, of which `entry` was made, comes from elsewhere (pinned
+    host memory: its copy may still be running when _as_device returns, and the
+    caller may refill the buffer once the call that uses it has returned)."""
+    for t, e in zip(w, entry):
+        if t is not e and t.device != dev:
+            return True
+    return False
 
 
 def _fp4_entry(w: tuple, dev: torch.device):
@@ -157,7 +160,7 @@ class FusedMoEFFN:
             else:
                 continue
             if ent is not w:  # (a ready entry is the loader's own)
-                wait = wait or _copied(w, dev)
+                wait = wait or _copied(w, ent, dev)
             entries[eid] = ent
         if inter is None:
             return torch.zeros_like(hidden_states)
@@ -185,7 +188,7 @@ class FusedMoEFFN:
             ent, kind = _fp4_entry(fp4_data[e], dev)
             entries.append(ent)
             kinds.add(kind)
-            wait = wait or _copied(fp4_data[e], dev)
+            wait = wait or _copied(fp4_data[e], ent, dev)
         if len(kinds) > 1:
             raise TypeError("experts of one call mix E8M0 and fp32 scales")
         table = ops.expert_table(entries, dev, wait=wait)
@@ -238,9 +241,8 @@ def fused_expert_ffn_pt(hidden: torch.Tensor, w1: torch.Tensor, w3: torch.Tensor
                         swiglu_limit: float = 10.0) -> torch.Tensor:
     """One bf16 expert (fused_moe.py:383-395) as a weight-1 slot of the HIP FFN."""
     dev = hidden.device
-    copied = _copied((w1, w3, w2), dev)
-    w1, w3, w2 = _bf16_entry((w1, w3, w2), dev)
-    table = ops.expert_table([(w1, w3, w2)], dev, wait=copied)
+    ent = _bf16_entry((w1, w3, w2), dev)
+    table = ops.expert_table([ent], dev, wait=_copied((w1, w3, w2), ent, dev))
     m = hidden.shape[0]
     idx = torch.zeros(m, 1, dtype=torch.int64, device=dev)
     w = torch.ones(m, 1, dtype=torch.float32, device=dev)
@@ -263,7 +265,7 @@ def fused_expert_ffn_triton(hidden: torch.Tensor, w1: torch.Tensor, w3: torch.Te
         given = (w1, w3, w2)
         ent, kind = _bf16_entry(given, dev), SCALE_E8M0
     inter = ent[0].shape[0]
-    table = ops.expert_table([ent], dev, wait=_copied(given, dev))
+    table = ops.expert_table([ent], dev, wait=_copied(given, ent, dev))
     m = hidden.shape[0]
     idx = torch.zeros(m, 1, dtype=torch.int64, device=dev)
     w = torch.ones(m, 1, dtype=torch.float32, device=dev)
