@@ -82,7 +82,8 @@ def _fp4_entry(w: tuple, dev: torch.device):
 
 
 def _bf16_entry(w: tuple, dev: torch.device):
-    return tuple(_as_device(t, dev).to(torch.bfloat16).contiguous() for t in w)
+    return tuple((t if t.dtype == torch.bfloat16 else t.to(torch.bfloat16)).contiguous()
+                 for t in (_as_device(t, dev) for t in w))
 
 
 def _run_decode_chunks(x: torch.Tensor, topk_idx: torch.Tensor, topk_w: torch.Tensor, table: torch.Tensor,

@@ -194,8 +194,9 @@ def expert_table(entries: list, device: torch.device, wait: bool = True) -> torc
     # wait: through pinned memory (torch's cached host allocator keeps it until
     # the copy is done).  A graph would read the host memory again when others
     # own it: refused under capture.
-    if torch.device(device).type == "cuda":
-        if _capturing(torch.device(device)):
+    device = torch.device(device)
+    if device.type == "cuda":
+        if _capturing(device):
             raise RuntimeError("an expert table is made from host memory: not under graph capture")
         if not wait:
             return rows.pin_memory().to(device, non_blocking=True)
